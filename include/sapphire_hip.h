@@ -96,9 +96,9 @@ int sapphire_gemm_bf16_dev(const void *w, int M, int K, const float *x, int ldx,
  * kernel_gemv_batch (dispatch.c:87-99, 234-266) for Q4_0/Q8_0, which the reference
  * itself rejects (pool.c:318-321); its meaning is `batch` independent kernel_gemv calls.
  * X and Y are row-major [batch][K] / [batch][M]. On the TILED layout the rows run on the
- * fp16 matrix cores, 16 sequences per pass (longer batches loop), with `ws` holding
- * sapphire_gemm_workspace_bytes(dtype, M, K) bytes of device memory (K-split partial
- * sums); calls that share a workspace must be ordered on one stream. On AOS/PACKED it is
+ * fp16 matrix cores, up to 16 sequences in one pass and longer batches in passes of 512, with
+ * `ws` holding sapphire_gemm_workspace_bytes(dtype, M, K) bytes of device memory (K-split
+ * partial sums, prepared activations); calls that share a workspace must be ordered on one stream. On AOS/PACKED it is
  * the vector kernel and ws may be NULL. */
 size_t sapphire_gemm_workspace_bytes(int dtype, int M, int K);
 int sapphire_gemm_q_dev(int dtype, int layout, const void *w, int M, int K, const float *X, int batch,

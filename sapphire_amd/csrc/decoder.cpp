@@ -957,8 +957,8 @@ sapphire_decoder_t *create_decoder(const sapphire_decoder_config_t *cfg, const s
         !hip_ok(hipDeviceSynchronize(), "greedy counters zero"))
         return fail();
     if (B > 1 || d->pf_ok) {
-        const size_t wsb = std::max({gemm_workspace_bytes(H, c.ffn), gemm_workspace_bytes(H, nq),
-                                     gemm_workspace_bytes(c.vocab, H)});
+        const size_t wsb = std::max({gemm_workspace_bytes(H, c.ffn, kGemmSeqs), gemm_workspace_bytes(H, nq, kGemmSeqs),
+                                     gemm_workspace_bytes(c.vocab, H, kGemmSeqs)});
         if (!dev_alloc(d, &d->gws, wsb, "gemm workspace")) return fail();
     }
     if (B > 1) {

@@ -142,7 +142,7 @@ int gemv_exec(kernel_context_t *c, const tensor_t *A, const float *X, float *Y, 
     const void *w = mm ? tensor_device_tiled(A, c->stream) : tensor_device_weights(A, &layout, c->stream);
     if (!w) return -1;
     const size_t xb = (size_t)batch * Kp * sizeof(float), yb = (size_t)batch * M * sizeof(float);
-    const size_t wsb = mm ? gemm_workspace_bytes(M, Kp) : 0;
+    const size_t wsb = mm ? gemm_workspace_bytes(M, Kp, batch) : 0;
     if (!ensure_staging(c, align256(xb) + align256(yb), align256(xb) + align256(yb) + wsb)) return -1;
     char *hb = static_cast<char *>(c->h_stage);
     char *db = static_cast<char *>(c->d_stage);

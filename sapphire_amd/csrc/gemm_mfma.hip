@@ -22,6 +22,7 @@
 // in the GEMM itself (last workgroup to finish) needs device-scope fences, i.e. L2
 // write-backs across the XCDs, which cost more than the extra launch.
 #include "gemm_body.h"
+#include "gemm_wide.h"
 
 namespace sapphire {
 
@@ -437,9 +438,12 @@ int gemm_splits(int K) {
     return nsplit;
 }
 
-size_t gemm_workspace_bytes(int M, int K) {
+size_t gemm_workspace_bytes(int M, int K, int batch) {
     const int nsplit = gemm_splits(K);
-    return amax_offset(M, nsplit) + kAmaxBytes;
+    const size_t narrow = amax_offset(M, nsplit) + kAmaxBytes;
+    if (batch <= kBatchMax || !gemm_wide_supported(K)) return narrow;
+    const int T = std::min(batch, kWidePass);
+    return std::max(narrow, gemm_wide_operand_bytes(T, K) + gemm_wide_parts_bytes(M, T));
 }
 
 int launch_sum_parts(const float *parts, int nparts, size_t stride, int batch, int M, float *y, int ldy,
@@ -499,6 +503,24 @@ int launch_gemm_tiled(int dt, const void *w, int M, int K, const float *X, int b
         set_error("batched GEMM: bad arguments (batch=%d K=%d ws=%p X=%p; K %% 128 == 0, ws 256-byte and X "
                   "16-byte aligned)", batch, K, ws, (const void *)X);
         return -1;
+    }
+    // more than one pass of 16: the many-vector kernel, up to kWidePass vectors a pass
+    if (batch > kBatchMax && gemm_wide_supported(K)) {
+        for (int b0 = 0; b0 < batch; b0 += kWidePass) {
+            const int T = std::min(kWidePass, batch - b0);
+            GemmIn in;
+            in.x = X + (size_t)b0 * K;
+            in.ldx = K;
+            WideOut out;
+            out.y = Y + (size_t)b0 * M;
+            out.ldy = M;
+            const int ks = gemm_wide_splits(dt, M, K, T);
+            if (ks > 1) out.parts = reinterpret_cast<float *>(static_cast<char *>(ws) + gemm_wide_operand_bytes(T, K));
+            if (launch_gemm_wide_prep(dt, in, K, T, ws, st) != 0 || launch_gemm_wide(dt, w, M, K, T, ws, out, st) != 0 ||
+                (ks > 1 && launch_sum_parts(out.parts, ks, (size_t)T * M, T, M, out.y, M, st) != 0))
+                return -1;
+        }
+        return 0;
     }
     // passes of 16 sequences share the workspace; the stream orders them
     for (int b0 = 0; b0 < batch; b0 += kBatchMax) {

@@ -135,9 +135,11 @@ int launch_gemv_tiled_greedy_slots(int dt, const void *w, int M, int K, const fl
 int launch_token_slots_settle(TokenSlots *slots, int vocab, int *log, int *done, const StopSet &stop, int *err,
                               hipStream_t s);
 // Batched GEMM on the TILED layout (gemm_mfma.hip): Y[b][r] = W[r] . X[b] for b < batch, 16
-// sequences per pass. ws: gemm_workspace_bytes(M, K) bytes of 256-byte aligned device memory
-// (the K-split partial sums). Calls sharing a workspace must be ordered.
-size_t gemm_workspace_bytes(int M, int K);
+// sequences per pass, or (gemm_wide.hip) kWidePass when the batch is longer. ws:
+// gemm_workspace_bytes(M, K, batch) bytes of 256-byte aligned device memory (the K-split partial
+// sums, the prepared operands). Calls sharing a workspace must be ordered.
+constexpr int kWidePass = 512;
+size_t gemm_workspace_bytes(int M, int K, int batch);
 int launch_gemm_tiled(int dt, const void *w, int M, int K, const float *X, int batch, float *Y, void *ws,
                       hipStream_t s);
 // Number of K chunks (partial sums) of a batched GEMM with inner dimension K.

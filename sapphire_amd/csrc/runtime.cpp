@@ -178,7 +178,7 @@ int sapphire_gemv_q_dev(int dt, int layout, const void *w, int M, int K, const f
 
 size_t sapphire_gemm_workspace_bytes(int dt, int M, int K) {
     if (!is_quant(dt) || M <= 0 || K <= 0 || K % kBlock != 0) return 0;
-    return gemm_workspace_bytes(M, K);
+    return gemm_workspace_bytes(M, K, kWidePass);
 }
 
 int sapphire_gemm_q_dev(int dt, int layout, const void *w, int M, int K, const float *X, int batch, float *Y,

@@ -1,0 +1,62 @@
+"""More than 16 activation vectors through one quantized matrix (gemm_wide.hip) against the
+float64 products of the dequantized weights, at the edges of its tiles: 32 tokens, 64 / 128 / 256
+rows, K chunks of 32 blocks, K splits, passes of 512 tokens.
+
+Tolerance: an output is a float32 sum of K products in chunks, each product with a relative error
+of at most 2^-21 (two fp16 terms), so |error| <= (2^-21 + 2 sqrt(K) 2^-24) sum |w x| with room for
+the order of the sums; a wrong or missing product is of the order of sum |w x| / K.
+"""
+import numpy as np
+import pytest
+
+from sapphire_amd import synth
+from tests.test_gemm_gpu import TILED, _gemm, _ref
+from tests.test_nonfinite_gpu import _matrix, _patterns, _same_special
+
+pytestmark = pytest.mark.gpu
+
+CASES = [                 # m, k, batch
+    (1, 128, 17),         # one row, one group, the first batch of the path
+    (16, 1024, 32),       # one tile, one whole chunk
+    (65, 1152, 33),       # a remainder of everything: chunk + one group, 32 + 1 tokens
+    (640, 2048, 64),      # K split
+    (1152, 6912, 100),    # K split, chunks cut by the split
+    (129, 8192, 31),      # the longest K
+    (130, 8320, 20),      # past it: passes of 16
+    (4111, 640, 512),     # the 128- and 256-row tiles, one full pass
+    (8192, 256, 300),
+    (384, 384, 513),      # two passes, the second of one token
+]
+
+
+@pytest.mark.parametrize("dtype", [synth.Q4_0, synth.Q8_0], ids=["q4_0", "q8_0"])
+@pytest.mark.parametrize("m,k,batch", CASES, ids=lambda v: str(v))
+def test_gemm_wide(hip, dtype, m, k, batch):
+    from sapphire_amd.device import QMatrix
+    print(f"wide gemm dtype={dtype} {m}x{k} batch={batch}", flush=True)
+    W = synth.quant_matrix(dtype, m, k, seed=51, tensor_id=m + k)
+    X = synth.normal_f32((batch, k), 51, batch)
+    X *= np.exp2(synth.rng(51, 9).integers(-20, 20, (batch, 1))).astype(np.float32)
+    X[batch // 2] = 0.0
+    X[0, k // 2] *= np.float32(4096.0)             # one chunk's range far from the others'
+    got = _gemm(hip, QMatrix(dtype, W, layout=TILED), X)
+    w = synth.unpack_ints(dtype, W).astype(np.float64) * np.repeat(W["scale"].astype(np.float64), 32, axis=1)
+    ref, mag = X.astype(np.float64) @ w.T, np.abs(X.astype(np.float64)) @ np.abs(w).T
+    bound = (2.0 ** -21 + 2.0 * np.sqrt(k) * 2.0 ** -24) * mag
+    assert np.all(np.abs(got - ref) <= bound), f"worst {np.max(np.abs(got - ref) / np.maximum(bound, 1e-300)):.2f} of the bound"
+
+
+@pytest.mark.parametrize("dtype", [synth.Q4_0, synth.Q8_0], ids=["q4_0", "q8_0"])
+@pytest.mark.parametrize("m,k", [(96, 1152), (80, 6912)])
+def test_gemm_wide_non_finite(hip, oracle, dtype, m, k):
+    """NaN and infinite activations (also with K split) give the oracle's special values, in
+    their own rows only."""
+    from sapphire_amd.device import QMatrix
+    W = _matrix(dtype, m, k, 52)
+    X = synth.normal_f32((40, k), 52, 5)
+    for b, x in zip((1, 17, 32, 39), _patterns(k, 53).values()):
+        X[b] = x
+    got = _gemm(hip, QMatrix(dtype, W, layout=TILED), X)
+    ref = _ref(oracle, dtype, W, X)
+    for b in range(40):
+        _same_special(got[b], ref[b])
