@@ -28,6 +28,8 @@
 #include "../../include/decoder.h"
 #include "../../include/rope.h"
 #include "decode_kernels.h"
+#include "gemm_wide.h"
+#include "prefill.h"
 #include "internal.h"
 
 using namespace sapphire;
@@ -117,6 +119,14 @@ struct sapphire_decoder {
     float *pf_qkv = nullptr, *pf_attn = nullptr, *pf_o = nullptr, *pf_g = nullptr;
     float *pf_dparts = nullptr, *pf_dout = nullptr, *pf_part = nullptr;
     int *pf_tok = nullptr;       // [kPrefillChunk] tokens, then [kPrefillChunk] positions
+    // longer prompts: passes of up to wp_tokens tokens through the many-vector GEMMs (gemm_wide.h)
+    // and the prompt attention (prefill.h); 0 when the shapes do not fit them
+    int wp_tokens = 0;
+    float *wp_resid[2] = {nullptr, nullptr};
+    float *wp_qkv = nullptr, *wp_q = nullptr, *wp_part = nullptr, *wp_o = nullptr, *wp_g = nullptr, *wp_down = nullptr;
+    float2 *wp_ms = nullptr;
+    void *wp_op = nullptr;       // the GEMMs' prepared operands
+    int *wp_tok = nullptr;       // [max_ctx] the prompt's tokens
     std::vector<hipGraph_t> pf_graph;          // per sequence: a full chunk's pass, captured once
     std::vector<hipGraphExec_t> pf_exec;
     // temperature sampling (temperature > 0): the draws of a generate call [max_ctx][B], the
@@ -590,6 +600,107 @@ int enqueue_layers_batch(sapphire_decoder *d, const BatchRun &r) {
     return cur;
 }
 
+// Tokens of one pass of a long prompt, and the shortest prompt that takes it.
+constexpr int kWideTokens = 1024;
+constexpr int kWideMinTokens = kPrefillChunk + 1;
+
+// T tokens of one sequence (d_tokens, positions pos0 ..) through the layers: every weight read
+// once per pass. The last layer only writes its K/V rows, the one result of a prefill.
+int enqueue_layers_wide(sapphire_decoder *d, const int *d_tokens, int T, int pos0, float *kc, float *vc) {
+    const auto &c = d->cfg;
+    hipStream_t s = d->stream;
+    const int H = c.hidden, hd = c.head_dim, nq = c.n_heads * hd, nqkv = nq + 2 * c.n_kv_heads * hd, dt = c.wdtype;
+    const size_t layer_kv = (size_t)c.n_kv_heads * c.max_ctx * hd;
+    if (dec_embed_batch(d->embed, H, c.vocab, sqrtf((float)H), d_tokens, T, d->wp_resid[0], s) != 0) return -1;
+    int cur = 0, down_parts = 1;
+    // y = W x: one product, or the partial sums of its K splits for the next input pass to add
+    auto product = [&](const void *w, int M, int K, float *y) {
+        const int ks = gemm_wide_splits(dt, M, K, T);
+        WideOut o;
+        o.y = y;
+        o.ldy = M;
+        if (ks > 1) o.parts = y;
+        return launch_gemm_wide(dt, w, M, K, T, d->wp_op, o, s) == 0 ? ks : -1;
+    };
+    auto parts_in = [&](const float *x, const float *parts, int n, const float *w_delta, const float *w_norm) {
+        GemmIn in;
+        in.x = x;
+        in.ldx = H;
+        in.parts = parts;
+        in.nparts = n;
+        in.ldp = H;
+        in.part_stride = (size_t)T * H;
+        in.w_delta = w_delta;
+        in.resid_out = d->wp_resid[1 - cur];
+        in.ldr = H;
+        in.w_norm = w_norm;
+        in.eps = c.eps;
+        return in;
+    };
+    for (int l = 0; l < c.n_layers; ++l) {
+        const Layer &L = d->layers[l];
+        const bool last = l + 1 == c.n_layers;
+        // previous layer's finalize (transformer.c:231-239) + attention pre-norm (attention.c:316-325)
+        GemmIn qi;
+        if (l == 0) {
+            qi.x = d->wp_resid[cur];
+            qi.ldx = H;
+            qi.w_norm = L.n_attn;
+            qi.eps = c.eps;
+        } else {
+            qi = parts_in(d->wp_resid[cur], d->wp_down, down_parts, d->layers[l - 1].n_ffn_post, L.n_attn);
+            cur = 1 - cur;
+        }
+        WideOut qo;
+        qo.y = d->wp_qkv;
+        qo.ldy = nqkv;
+        if (launch_gemm_wide_prep(dt, qi, H, T, d->wp_op, s) != 0 ||
+            launch_gemm_wide(dt, L.t_qkv, nqkv, H, T, d->wp_op, qo, s) != 0)
+            return -1;
+        PrefillAttn at;
+        at.qkv = d->wp_qkv;
+        at.qn = L.qn;
+        at.kn = L.kn;
+        at.cos_t = L.global ? d->cos_g : d->cos_l;
+        at.sin_t = L.global ? d->sin_g : d->sin_l;
+        at.kc = kc + (size_t)l * layer_kv;
+        at.vc = vc + (size_t)l * layer_kv;
+        at.T = T;
+        at.pos0 = pos0;
+        at.nh = c.n_heads;
+        at.nkv = c.n_kv_heads;
+        at.hd = hd;
+        at.max_ctx = c.max_ctx;
+        at.window = L.global ? 0 : c.sliding_window > 0 ? c.sliding_window : 1024;
+        at.scale = 1.0f / sqrtf(c.query_pre_attn_scalar > 0.f ? c.query_pre_attn_scalar : (float)hd);
+        at.eps = c.eps;
+        at.part = last ? nullptr : d->wp_part;
+        at.ms = d->wp_ms;
+        int pieces = 0;
+        if (launch_prefill_attention(at, d->wp_q, &pieces, s) != 0) return -1;
+        if (last) break;
+        if (launch_gemm_wide_prep_attn(dt, d->wp_part, d->wp_ms, pieces, c.n_heads, hd, T, d->wp_op, s) != 0) return -1;
+        const int o_parts = product(L.t_o, H, nq, d->wp_o);
+        if (o_parts < 0) return -1;
+        // post-attention norm + residual (attention.c:356-366), FFN pre-norm (transformer.c:119-121)
+        const GemmIn fi = parts_in(d->wp_resid[cur], d->wp_o, o_parts, L.n_attn_post, L.n_ffn);
+        cur = 1 - cur;
+        WideOut fo;
+        fo.y = d->wp_g;
+        fo.ldy = c.ffn;
+        fo.geglu = true;
+        GemmIn di;
+        di.x = d->wp_g;
+        di.ldx = c.ffn;
+        if (launch_gemm_wide_prep(dt, fi, H, T, d->wp_op, s) != 0 ||
+            launch_gemm_wide(dt, L.t_gu, 2 * c.ffn, H, T, d->wp_op, fo, s) != 0 ||
+            launch_gemm_wide_prep(dt, di, c.ffn, T, d->wp_op, s) != 0 ||
+            (down_parts = product(L.t_down, H, c.ffn, d->wp_down)) < 0)
+            return -1;
+    }
+    return 0;
+}
+
 // One step of the batched decoder, enqueued on d->stream (recorded into the graph).
 int enqueue_step_batch(sapphire_decoder *d) {
     const auto &c = d->cfg;
@@ -989,6 +1100,24 @@ sapphire_decoder_t *create_decoder(const sapphire_decoder_config_t *cfg, const s
             !dev_alloc_t(d, &d->pf_part, p * attn_part_floats(c.n_heads, hd), "prefill attention partials") ||
             !dev_alloc_t(d, &d->pf_tok, 2 * p, "prefill tokens"))
             return fail();
+    }
+    if (d->pf_ok && prefill_attn_supported(c.n_heads, c.n_kv_heads, hd) && gemm_wide_supported(H) &&
+        gemm_wide_supported(nq) && gemm_wide_supported(c.ffn) && c.max_ctx >= kWideMinTokens) {
+        const int T = std::min(kWideTokens, c.max_ctx);
+        const size_t t = (size_t)T, rows = t * c.n_heads * kPrefillPieces;
+        // a product's result, or the partial sums of its K splits
+        const size_t hp = std::max(t * H, gemm_wide_parts_bytes(H, T) / sizeof(float));
+        const size_t ob = std::max({gemm_wide_operand_bytes(T, H), gemm_wide_operand_bytes(T, nq),
+                                    gemm_wide_operand_bytes(T, c.ffn)});
+        if (!dev_alloc_t(d, &d->wp_resid[0], t * H, "prompt resid") ||
+            !dev_alloc_t(d, &d->wp_resid[1], t * H, "prompt resid") ||
+            !dev_alloc_t(d, &d->wp_qkv, t * (nq + 2 * nk), "prompt qkv") || !dev_alloc_t(d, &d->wp_q, t * nq, "prompt q") ||
+            !dev_alloc_t(d, &d->wp_part, rows * hd, "prompt attention partials") ||
+            !dev_alloc_t(d, &d->wp_ms, rows, "prompt attention maxima") || !dev_alloc_t(d, &d->wp_o, hp, "prompt o") ||
+            !dev_alloc_t(d, &d->wp_g, t * c.ffn, "prompt g") || !dev_alloc_t(d, &d->wp_down, hp, "prompt down") ||
+            !dev_alloc(d, &d->wp_op, ob, "prompt operands") || !dev_alloc_t(d, &d->wp_tok, c.max_ctx, "prompt tokens"))
+            return fail();
+        d->wp_tokens = T;
     }
     if (B == 1 && !setup_persistent(d)) return fail();
     // the zero fills above run on the null stream; the decoder's stream does not wait for it
@@ -1390,7 +1519,19 @@ int sapphire_decoder_prefill(sapphire_decoder_t *d, int seq, const int *tokens, 
         SPH_CHECK(hipEventRecord(e0, d->stream));
     }
     const size_t seq_kv = (size_t)c.n_layers * c.n_kv_heads * c.max_ctx * c.head_dim;
-    for (int k = 0; k < nchunks; ++k) {
+    const bool wide = d->wp_tokens > 0 && n >= kWideMinTokens;
+    if (wide) {
+        SPH_CHECK(hipMemcpyAsync(d->wp_tok, tokens, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, d->stream));
+        // passes of equal length
+        const int passes = (n + d->wp_tokens - 1) / d->wp_tokens;
+        for (int k = 0; k < passes; ++k) {
+            const int c0 = (int)((long)k * n / passes), c1 = (int)((long)(k + 1) * n / passes);
+            if (enqueue_layers_wide(d, d->wp_tok + c0, c1 - c0, pos + c0, d->kc + (size_t)seq * seq_kv,
+                                    d->vc + (size_t)seq * seq_kv) != 0)
+                return -1;
+        }
+    }
+    for (int k = 0; k < (wide ? 0 : nchunks); ++k) {
         const int c0 = k * kPrefillChunk, m = std::min(kPrefillChunk, n - c0);
         int *h = host.data() + (size_t)k * 2 * kPrefillChunk;
         for (int i = 0; i < m; ++i) {

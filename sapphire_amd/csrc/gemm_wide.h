@@ -19,6 +19,10 @@ size_t gemm_wide_parts_bytes(int M, int T);
 // The operands of T tokens from `in` (GemmIn's transform, sums of squares as trees).
 int launch_gemm_wide_prep(int dt, const GemmIn &in, int K, int T, void *operand, hipStream_t s);
 
+// The same from the attention's partials (prefill.h), K = nh * hd.
+int launch_gemm_wide_prep_attn(int dt, const float *part, const void *ms, int pieces, int nh, int hd, int T,
+                               void *operand, hipStream_t s);
+
 // y[t * ldy + r], or with geglu y[t * ldy + j] = gelu(gate_j) * up_j of rows interleaved by
 // eight; parts set: the K splits' partial sums [split][T][M] instead (gemm_wide_splits of them).
 struct WideOut {

@@ -47,11 +47,19 @@ Operand operand_at(void *buf, int T, int K) {
     return o;
 }
 
+constexpr int kAttnPieces = 8;
+struct AttnParts {
+    const float *part;             // [pieces][T][nh][hd], unnormalised
+    const float2 *ms;              // [pieces][T][nh]: maximum (log2 units), sum
+    int pieces, hd;
+};
+
 // grid (tokens): token t's input transform (GemmIn's: sum of parts, rmsnorm_delta, residual,
 // pre-norm; sums of squares as trees), the range scale over the finite values, the non-finite
 // record and the hi / lo split. Thread p takes the pairs p + 256 i (8 activations each).
-template <int DT, int NP>
-__global__ __launch_bounds__(kThreads) void gemm_wide_prep_kernel(GemmIn in, int K, Operand op) {
+// ATTN: the input is the merge of the attention's partials instead (nh = K / hd heads).
+template <int DT, int NP, bool ATTN = false>
+__global__ __launch_bounds__(kThreads) void gemm_wide_prep_kernel(GemmIn in, int K, Operand op, AttnParts at = {}) {
     __shared__ float wsq[2][kWavesWg];
     __shared__ float wmx[NP][kWavesWg];
     __shared__ int wfl[kWavesWg];
@@ -110,6 +118,40 @@ __global__ __launch_bounds__(kThreads) void gemm_wide_prep_kernel(GemmIn in, int
             for (int i = 0; i < NP; ++i)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[i][e] = __fadd_rn(xv[i][e], v[i][e]);
+    }
+    if constexpr (ATTN) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int p = tid + i * kThreads;
+            if (p >= pairs) continue;
+            const int nh = K / at.hd, h = p * 8 / at.hd, d = p * 8 - h * at.hd;
+            const size_t row = (size_t)t * nh + h, rows = (size_t)gridDim.x * nh;
+            // every piece's loads first; a piece without positions (-inf, 0) has no O
+            float2 ms[kAttnPieces];
+            float ov[kAttnPieces][8];
+#pragma unroll
+            for (int c = 0; c < kAttnPieces; ++c) {
+                ms[c] = make_float2(-INFINITY, 0.f);
+                if (c < at.pieces) {
+                    ms[c] = at.ms[c * rows + row];
+                    load8(at.part + (c * rows + row) * at.hd + d, ov[c]);
+                }
+            }
+            float top = -INFINITY, sum = 0.f;
+#pragma unroll
+            for (int c = 0; c < kAttnPieces; ++c)
+                if (ms[c].y != 0.f) top = fmaxf(top, ms[c].x);
+#pragma unroll
+            for (int c = 0; c < kAttnPieces; ++c)
+                if (ms[c].y != 0.f) {
+                    const float f = __builtin_amdgcn_exp2f(ms[c].x - top);
+                    sum = __fadd_rn(sum, __fmul_rn(ms[c].y, f));
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[i][e] = __builtin_fmaf(ov[c][e], f, v[i][e]);
+                }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[i][e] = __fdiv_rn(v[i][e], sum);
+        }
     }
     if (in.resid_out)
 #pragma unroll
@@ -481,8 +523,21 @@ int launch_gemm_wide_prep(int dt, const GemmIn &in, int K, int T, void *operand,
     const bool small = K <= 8 * kThreads;
     auto kern = dt == DT_Q4_0 ? (small ? gemm_wide_prep_kernel<DT_Q4_0, 1> : gemm_wide_prep_kernel<DT_Q4_0, 4>)
                               : (small ? gemm_wide_prep_kernel<DT_Q8_0, 1> : gemm_wide_prep_kernel<DT_Q8_0, 4>);
-    hipLaunchKernelGGL(kern, dim3(T), dim3(kThreads), 0, st, in, K, op);
+    hipLaunchKernelGGL(kern, dim3(T), dim3(kThreads), 0, st, in, K, op, AttnParts{});
     return hip_ok(hipGetLastError(), "gemm_wide prep launch") ? 0 : -1;
+}
+
+int launch_gemm_wide_prep_attn(int dt, const float *part, const void *ms, int pieces, int nh, int hd, int T,
+                               void *operand, hipStream_t st) {
+    const int K = nh * hd;
+    if (!gemm_wide_supported(K) || K > 8 * kThreads || T <= 0 || pieces < 1 || pieces > kAttnPieces || hd % 8 != 0) {
+        set_error("wide GEMM attention input: unsupported arguments (T=%d, %d heads of %d, %d pieces)", T, nh, hd, pieces);
+        return -1;
+    }
+    const AttnParts at{part, static_cast<const float2 *>(ms), pieces, hd};
+    auto kern = dt == DT_Q4_0 ? gemm_wide_prep_kernel<DT_Q4_0, 1, true> : gemm_wide_prep_kernel<DT_Q8_0, 1, true>;
+    hipLaunchKernelGGL(kern, dim3(T), dim3(kThreads), 0, st, GemmIn{}, K, operand_at(operand, T, K), at);
+    return hip_ok(hipGetLastError(), "gemm_wide attention prep launch") ? 0 : -1;
 }
 
 int launch_gemm_wide(int dt, const void *w, int M, int K, int T, const void *operand, const WideOut &out,
