@@ -15,10 +15,13 @@
 //   is one pair (d0, d1) for a given binade. The binades a chain can occupy at a sub-chunk's
 //   start are fixed to at most two by the exact prefix sum and the error bound of recursive
 //   summation (|fl-sum - sum| <= n 2^-24 sum for nonnegative terms);
-// * one wave per row walks the sub-chunks with these maps, 64 at a time, and in a sub-chunk
-//   where the binade changes or the draw is reached scans its lanes' maps (16 elements each)
-//   to find the lane where that happens; that lane adds its elements with real float adds
-//   (the reference's own operation).
+// * the maps are kept for groups of 64 elements as well, each for the binades of its own start;
+// * one wave per row walks the sub-chunks with these maps, 64 at a time; in a sub-chunk where
+//   the binade changes or the draw is reached it scans the 16 groups' maps, and the group where
+//   that happens is added element by element with real float adds (the reference's own
+//   operation), whatever binades it crosses. (Composing 16 elements' maps per lane in the walk
+//   instead, once per binade change, took 107 us per walk of 262144 weights; a group's 64 adds
+//   take a third of a microsecond, and the walk 37 us.)
 // The weights come from libm_expf, glibc's expf bit for bit.
 #include "internal.h"
 #include "libm_expf.h"
@@ -32,7 +35,9 @@ constexpr int kWave = 64;
 constexpr int kThreads = 256;
 constexpr int kPer = 4;                         // elements per thread in the grid kernels
 constexpr int kSub = kThreads * kPer;           // elements per sub-chunk (one grid workgroup)
-constexpr int kRun = kSub / kWave;              // consecutive elements per lane in the walk
+constexpr int kGroup = kWave;                   // elements per group
+constexpr int kGroups = kSub / kGroup;          // groups per sub-chunk: one per row of 16 lanes
+static_assert(kGroup == 16 * kPer && kGroups == 16, "a group is a row of 16 lanes of the grid kernels");
 constexpr int kMaxSubs = 2048;                  // n <= 2^21 keeps the error bound below 1/4
 constexpr int kCap = 1 << 28;                   // saturation of map increments
 constexpr int kZero = -1000, kSub_ = -127;      // binade ids of 0 and of the subnormals
@@ -44,7 +49,7 @@ struct SubStat {         // per row and sub-chunk
     int nan0;            // sub-chunk 0 only: whether the row's first scaled logit is NaN
     double wsum;         // sum of the sub-chunk's weights (exact enough for the bounds)
 };
-struct SubMaps {         // per row and sub-chunk: its map for the chunk's (up to) two binades
+struct SubMaps {         // per row and sub-chunk or group: its map for its (up to) two binades
     int reg[2];
     int d[2][2];
 };
@@ -65,21 +70,22 @@ __device__ __forceinline__ Reg reg_id(int id) {
     if (id == kSub_) return {kSub_, -149, 1 << 23};
     return {id, id - 23, 1 << 24};
 }
-__device__ __forceinline__ Reg reg_of(float v) {
-    if (v == 0.0f) return reg_zero();
-    if (v < 0x1p-126f) return reg_id(kSub_);
-    return reg_id(ilogbf(v));
+__device__ __forceinline__ Reg reg_of(float v) {               // v >= +0, finite
+    const int e = (int)(__float_as_uint(v) >> 23);
+    return v == 0.0f ? reg_zero() : reg_id(e == 0 ? kSub_ : e - 127);
 }
 __device__ __forceinline__ Reg reg_of_bound(double x) {
     if (!(x > 0.0)) return reg_zero();
     if (x < 0x1p-126) return reg_id(kSub_);
     return reg_id(min(ilogb(x), 127));
 }
-__device__ __forceinline__ int m_of(float v, const Reg &R) {
-    return R.id == kZero ? 0 : (int)ldexp((double)v, -R.uexp);
+__device__ __forceinline__ int m_of(float v, const Reg &R) {    // v in R
+    const int f = (int)(__float_as_uint(v) & 0x7fffffu);
+    return R.id == kZero ? 0 : R.id == kSub_ ? f : f | 0x800000;
 }
 __device__ __forceinline__ float val_of(int M, const Reg &R) {   // exact for M < R.mlim
-    return R.id == kZero ? 0.0f : (float)ldexp((double)M, R.uexp);
+    const uint32_t f = (uint32_t)M & 0x7fffffu;
+    return R.id == kZero ? 0.0f : __uint_as_float(R.id == kSub_ ? f : (uint32_t)(R.id + 127) << 23 | f);
 }
 
 struct Map {
@@ -259,79 +265,6 @@ __device__ __forceinline__ uint32_t chain_elem(float wv, int chain, float sum) {
     return __float_as_uint(chain ? __fdiv_rn(wv, sum) : wv);
 }
 
-// Ordered composition of the block's per-thread maps; the result in thread 0.
-__device__ Map block_compose(Map m, Map *sh) {
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        Map o;
-        o.d0 = __shfl_down(m.d0, off, kWave);
-        o.d1 = __shfl_down(m.d1, off, kWave);
-        if ((lane & (2 * off - 1)) == 0 && lane + off < kWave) m = compose(m, o);
-    }
-    if (lane == 0) sh[wid] = m;
-    __syncthreads();
-    if (threadIdx.x == 0)
-        for (int k = 1; k < kThreads / kWave; ++k) m = compose(m, sh[k]);
-    return m;
-}
-
-// grid (sub-chunks, batch): each sub-chunk's map (chain 0: the weight sum; chain 1: the
-// running sum of the weights over the float sum) for the binades the chain can be in at the
-// sub-chunk's start.
-__global__ __launch_bounds__(kThreads) void smp_maps(const float *__restrict__ w, int n, size_t ldw, int chain,
-                                                     const SubStat *__restrict__ stats,
-                                                     const RowInfo *__restrict__ rows, SubMaps *__restrict__ maps) {
-    __shared__ double sd[kThreads / kWave];
-    __shared__ Map sm[2][kThreads / kWave];
-    const int nsub = gridDim.x, q = blockIdx.x, b = blockIdx.y;
-    const RowInfo ri = rows[b];
-    if (ri.bad) return;
-    const SubStat *st = stats + (size_t)b * nsub;
-    // the exact sum of the weights before this sub-chunk
-    double p = 0.0;
-    for (int k = threadIdx.x; k < q; k += kThreads) p += st[k].wsum;
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) p += __shfl_xor(p, off, kWave);
-    if ((threadIdx.x & (kWave - 1)) == 0) sd[threadIdx.x / kWave] = p;
-    __syncthreads();
-    p = sd[0];
-    for (int k = 1; k < kThreads / kWave; ++k) p += sd[k];
-    // recursive summation of n nonnegative floats: relative error below (n + 2) 2^-24 (with
-    // margin); the quotients w / sum add 2^-24 relative each, and subnormal ones 2^-150
-    double rel = 2.0 * (n + 2) * 0x1p-24, abs_err = 0.0;
-    if (chain) {
-        p /= (double)ri.sum;
-        rel += 0x1p-22;
-        abs_err = (double)n * 0x1p-149;
-    }
-    const Reg lo = reg_of_bound(p * (1.0 - rel) - abs_err), hi = reg_of_bound(p * (1.0 + rel) + abs_err);
-    const float *wr = w + (size_t)b * ldw;
-    const int i0 = q * kSub + threadIdx.x * kPer;
-    Map m0 = map_id(), m1 = map_id();
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const int i = i0 + k;
-        if (i < n) {
-            const uint32_t x = chain_elem(wr[i], chain, ri.sum);
-            m0 = compose(m0, elem_map(x, lo));
-            m1 = compose(m1, elem_map(x, hi));
-        }
-    }
-    m0 = block_compose(m0, sm[0]);
-    m1 = block_compose(m1, sm[1]);
-    if (threadIdx.x == 0) {
-        SubMaps cm;
-        cm.reg[0] = lo.id;
-        cm.d[0][0] = m0.d0;
-        cm.d[0][1] = m0.d1;
-        cm.reg[1] = hi.id;
-        cm.d[1][0] = m1.d0;
-        cm.d[1][1] = m1.d1;
-        maps[(size_t)b * nsub + q] = cm;
-    }
-}
-
 // One DPP move of both halves of a map; lanes without a source (and rows outside row_mask)
 // read 0, the identity map.
 template <int CTRL, int ROW_MASK>
@@ -340,14 +273,19 @@ __device__ __forceinline__ Map dpp_map(Map m) {
             __builtin_amdgcn_update_dpp(0, m.d1, CTRL, ROW_MASK, 0xf, true)};
 }
 
+// Inclusive scan of the maps of each row of 16 lanes.
+__device__ __forceinline__ Map row_scan(Map m) {
+    m = compose(dpp_map<0x111, 0xf>(m), m);   // row_shr:1
+    m = compose(dpp_map<0x112, 0xf>(m), m);   // row_shr:2
+    m = compose(dpp_map<0x114, 0xf>(m), m);   // row_shr:4
+    return compose(dpp_map<0x118, 0xf>(m), m);   // row_shr:8
+}
+
 // Inclusive scan of the wave's maps in lane order (lane l gets m_0 ... m_l composed): shifts
 // by 1, 2, 4, 8 within each 16-lane row, then the last lane of row 0 (and of row 2) into the
 // next row, then lane 31 into rows 2 and 3.
 __device__ __forceinline__ Map wave_scan(Map m) {
-    m = compose(dpp_map<0x111, 0xf>(m), m);   // row_shr:1
-    m = compose(dpp_map<0x112, 0xf>(m), m);   // row_shr:2
-    m = compose(dpp_map<0x114, 0xf>(m), m);   // row_shr:4
-    m = compose(dpp_map<0x118, 0xf>(m), m);   // row_shr:8
+    m = row_scan(m);
     m = compose(dpp_map<0x142, 0xa>(m), m);   // row_bcast:15 into rows 1 and 3
     m = compose(dpp_map<0x143, 0xc>(m), m);   // row_bcast:31 into rows 2 and 3
     return m;
@@ -355,20 +293,115 @@ __device__ __forceinline__ Map wave_scan(Map m) {
 
 __device__ __forceinline__ int first_lane(unsigned long long bal) { return __builtin_ctzll(bal); }
 
+// The binades a chain can be in after weights of exact sum p (chain 1: over the float sum), at
+// most two. Recursive summation of n nonnegative floats: relative error below (n + 2) 2^-24
+// (with margin); the quotients w / sum add 2^-24 relative each, and subnormal ones 2^-150.
+__device__ __forceinline__ void chain_regs(double p, int n, int chain, float sum, Reg &lo, Reg &hi) {
+    double rel = 2.0 * (n + 2) * 0x1p-24, abs_err = 0.0;
+    if (chain) {
+        p /= (double)sum;
+        rel += 0x1p-22;
+        abs_err = (double)n * 0x1p-149;
+    }
+    lo = reg_of_bound(p * (1.0 - rel) - abs_err);
+    hi = reg_of_bound(p * (1.0 + rel) + abs_err);
+}
+
+// The map of binade id in a group or sub-chunk; one that cannot be applied (and ends the scan
+// there) when it was not prepared.
+__device__ __forceinline__ Map map_for(const SubMaps &c, int id) {
+    const int k = c.reg[0] == id ? 0 : (c.reg[1] == id ? 1 : -1);
+    return k < 0 ? Map{kCap, kCap} : Map{c.d[k][0], c.d[k][1]};
+}
+
+// grid (sub-chunks, batch): the maps (chain 0: the weight sum; chain 1: the running sum of the
+// weights over the float sum) of each group for the binades the chain can be in at its start,
+// and of the sub-chunk for those at its own. A sub-chunk that stays in one binade has that
+// binade prepared in every group, so its map is the groups' maps composed.
+__global__ __launch_bounds__(kThreads) void smp_maps(const float *__restrict__ w, int n, size_t ldw, int chain,
+                                                     const SubStat *__restrict__ stats,
+                                                     const RowInfo *__restrict__ rows, SubMaps *__restrict__ maps,
+                                                     SubMaps *__restrict__ gmaps) {
+    __shared__ double sd[kThreads / kWave], sg[kGroups];
+    __shared__ SubMaps gm[kGroups];
+    const int nsub = gridDim.x, q = blockIdx.x, b = blockIdx.y;
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave, g = threadIdx.x / 16;
+    const float *wr = w + (size_t)b * ldw;
+    const int i0 = q * kSub + threadIdx.x * kPer;
+    float wv[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) wv[k] = i0 + k < n ? wr[i0 + k] : 0.0f;
+    const RowInfo ri = rows[b];
+    if (ri.bad) return;
+    const SubStat *st = stats + (size_t)b * nsub;
+    // the exact sums of the weights before this sub-chunk, and of its groups
+    double p = 0.0, gs = 0.0;
+    for (int k = threadIdx.x; k < q; k += kThreads) p += st[k].wsum;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) gs += (double)wv[k];
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) p += __shfl_xor(p, off, kWave);
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) gs += __shfl_xor(gs, off, kWave);
+    if (lane == 0) sd[wid] = p;
+    if ((lane & 15) == 0) sg[g] = gs;
+    __syncthreads();
+    p = sd[0];
+    for (int k = 1; k < kThreads / kWave; ++k) p += sd[k];
+    double pg = p;
+#pragma unroll
+    for (int k = 0; k < kGroups - 1; ++k) pg += k < g ? sg[k] : 0.0;
+    Reg lo, hi;
+    chain_regs(pg, n, chain, ri.sum, lo, hi);
+    Map m0 = map_id(), m1 = map_id();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const uint32_t x = chain_elem(wv[k], chain, ri.sum);
+        m0 = compose(m0, elem_map(x, lo));
+        m1 = compose(m1, elem_map(x, hi));
+    }
+    // the row of 16 lanes composed in order, into its last lane
+    m0 = row_scan(m0);
+    m1 = row_scan(m1);
+    if ((lane & 15) == 15) {
+        SubMaps c;
+        c.reg[0] = lo.id;
+        c.d[0][0] = m0.d0;
+        c.d[0][1] = m0.d1;
+        c.reg[1] = hi.id;
+        c.d[1][0] = m1.d0;
+        c.d[1][1] = m1.d1;
+        gm[g] = c;
+        gmaps[((size_t)b * nsub + q) * kGroups + g] = c;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        Reg sl, sh;
+        chain_regs(p, n, chain, ri.sum, sl, sh);
+        const int id = threadIdx.x == 0 ? sl.id : sh.id;
+        Map m = map_id();
+        for (int k = 0; k < kGroups; ++k) m = compose(m, map_for(gm[k], id));
+        SubMaps &c = maps[(size_t)b * nsub + q];
+        c.reg[threadIdx.x] = id;
+        c.d[threadIdx.x][0] = m.d0;
+        c.d[threadIdx.x][1] = m.d1;
+    }
+}
+
 // grid (batch), one wave per row: the chain walk. chain 0 stores the float sum of the weights
 // in RowInfo; chain 1 finds the first index whose running sum reaches the row's draw r
 // (draws[step * batch + b], step = *d_step or 0) and writes the token (n - 1 if none, or for
 // a bad row). The wave takes 64 sub-chunks at a time, one per lane: a scan of their maps in
 // the chain's binade finds the first sub-chunk in which the binade changes or r is reached
-// (or whose binades were not prepared). In that sub-chunk each lane holds 16 consecutive
-// elements, a scan of the lanes' maps finds the first lane where the same happens, and that
-// lane adds its elements with real float adds; the scan resumes after it.
+// (or whose binades were not prepared). There a scan of the 16 groups' maps finds the first
+// group where the same happens, and its elements are added one by one; the scan resumes after it.
 __global__ __launch_bounds__(kWave) void smp_walk(const float *__restrict__ w, int n, size_t ldw, int chain,
                                                   int nsub, const SubMaps *__restrict__ maps,
-                                                  RowInfo *__restrict__ rows, const float *__restrict__ draws,
-                                                  const int *__restrict__ d_step, int batch,
-                                                  int *__restrict__ tokens) {
+                                                  const SubMaps *__restrict__ gmaps, RowInfo *__restrict__ rows,
+                                                  const float *__restrict__ draws, const int *__restrict__ d_step,
+                                                  int batch, int *__restrict__ tokens) {
     __shared__ SubMaps cm[kMaxSubs];
+    __shared__ float xs[kSub];
     const int b = blockIdx.x, lane = threadIdx.x;
     const RowInfo ri = rows[b];
     if (ri.bad) {
@@ -386,73 +419,62 @@ __global__ __launch_bounds__(kWave) void smp_walk(const float *__restrict__ w, i
         {
             const Reg R = reg_of(v);
             const int M0 = m_of(v, R), qi = q + lane;
-            Map m = map_id();
-            if (qi < nsub) {
-                const SubMaps &c = cm[qi];
-                const int k = c.reg[0] == R.id ? 0 : (c.reg[1] == R.id ? 1 : -1);
-                m = k < 0 ? Map{kCap, kCap} : Map{c.d[k][0], c.d[k][1]};
-            }
+            const Map m = qi < nsub ? map_for(cm[min(qi, nsub - 1)], R.id) : map_id();
             const int Me = apply(M0, wave_scan(m));
             const bool stop = qi < nsub && (Me >= R.mlim || r <= val_of(Me, R));
             const unsigned long long bal = __ballot(stop);
             if (bal == 0) {
                 const int last = min(kWave, nsub - q) - 1;
-                v = val_of(__shfl(Me, last, kWave), R);
+                v = val_of(__builtin_amdgcn_readlane(Me, last), R);
                 q += kWave;
                 continue;
             }
             const int s = first_lane(bal);
-            const int Mprev = __shfl(Me, s > 0 ? s - 1 : 0, kWave);
-            if (s > 0) v = val_of(Mprev, R);
+            if (s > 0) v = val_of(__builtin_amdgcn_readlane(Me, s - 1), R);
             q += s;
         }
-        // sub-chunk q element by element: lane l holds elements base + 16 l .. + 15
-        const int base = q * kSub, e0 = base + lane * kRun;
-        uint32_t x[kRun];
+        // sub-chunk q: lane g < 16 holds group g's maps; the elements go to LDS
+        const int base = q * kSub;
+        const SubMaps gm = gmaps[((size_t)b * nsub + q) * kGroups + (lane & (kGroups - 1))];
+        float x[kGroups];
 #pragma unroll
-        for (int j = 0; j < kRun; ++j) {
-            const int i = e0 + j;
-            x[j] = i < n ? chain_elem(wr[i], chain, ri.sum) : 0u;
-        }
-        const int nval = max(0, min(kRun, n - e0));   // this lane's elements
-        int from = 0;                                  // the first lane not yet added
-        while (from < kWave) {
+        for (int g = 0; g < kGroups; ++g) x[g] = wr[min(base + g * kGroup + lane, n - 1)];
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) xs[g * kGroup + lane] = base + g * kGroup + lane < n ? x[g] : 0.0f;
+        __syncthreads();
+        int from = 0;                                  // the first group not yet added
+        while (from < kGroups) {
             const Reg R = reg_of(v);
             const int M0 = m_of(v, R);
-            Map m = map_id();
-            if (lane >= from)
-#pragma unroll
-                for (int j = 0; j < kRun; ++j)
-                    if (j < nval) m = compose(m, elem_map(x[j], R));
-            const int Me = apply(M0, wave_scan(m));
-            const bool stop = lane >= from && nval > 0 && (Me >= R.mlim || r <= val_of(Me, R));
+            const Map m = lane >= from && lane < kGroups ? map_for(gm, R.id) : map_id();
+            const int Me = apply(M0, row_scan(m));
+            const bool stop = lane >= from && lane < kGroups && (Me >= R.mlim || r <= val_of(Me, R));
             const unsigned long long bal = __ballot(stop);
             if (bal == 0) {                            // the rest of the sub-chunk stays in the binade
-                const unsigned long long has = __ballot(nval > 0);
-                const int last = has ? 63 - __builtin_clzll(has) : -1;
-                if (last >= from) v = val_of(__shfl(Me, last, kWave), R);
+                v = val_of(__builtin_amdgcn_readlane(Me, kGroups - 1), R);
                 break;
             }
             const int s = first_lane(bal);
-            const int Mprev = __shfl(Me, s > 0 ? s - 1 : 0, kWave);
-            float vv = s > from ? val_of(Mprev, R) : v;
-            int fnd = -1;
-            if (lane == s) {
+            if (s > from) v = val_of(__builtin_amdgcn_readlane(Me, s - 1), R);
+            // the group's 64 real adds (elements past the row are 0), every lane alike; if the
+            // draw is reached, again with lane j keeping the sum after element j
+            const int xb = (int)chain_elem(xs[s * kGroup + lane], chain, ri.sum);
+            const float v0 = v;
 #pragma unroll
-                for (int j = 0; j < kRun; ++j)
-                    if (j < nval && fnd < 0) {
-                        vv = __fadd_rn(vv, __uint_as_float(x[j]));
-                        if (r <= vv) fnd = e0 + j;
-                    }
-            }
-            v = __shfl(vv, s, kWave);
-            fnd = __shfl(fnd, s, kWave);
-            if (fnd >= 0) {
-                found = fnd;
+            for (int j = 0; j < kGroup; ++j) v = __fadd_rn(v, __int_as_float(__builtin_amdgcn_readlane(xb, j)));
+            if (r <= v) {
+                float c = v0, mine = 0.0f;
+#pragma unroll
+                for (int j = 0; j < kGroup; ++j) {
+                    c = __fadd_rn(c, __int_as_float(__builtin_amdgcn_readlane(xb, j)));
+                    mine = lane == j ? c : mine;
+                }
+                found = base + s * kGroup + first_lane(__ballot(r <= mine));
                 break;
             }
             from = s + 1;
         }
+        __syncthreads();
         ++q;
     }
     if (lane == 0) {
@@ -493,7 +515,8 @@ int subs_of(int n) { return (n + kSub - 1) / kSub; }
 
 size_t sample_workspace_bytes(int n, int batch) {
     const size_t cells = (size_t)subs_of(n) * batch;
-    return align256(cells * sizeof(SubStat)) + 2 * align256(cells * sizeof(SubMaps)) +
+    return align256(cells * sizeof(SubStat)) + align256(cells * sizeof(SubMaps)) +
+           align256(cells * kGroups * sizeof(SubMaps)) +
            align256((size_t)batch * sizeof(RowInfo));
 }
 
@@ -510,10 +533,10 @@ int launch_sample(const float *logits, int n, int batch, size_t ld, float temper
     char *p = static_cast<char *>(ws);
     auto *stats = reinterpret_cast<SubStat *>(p);
     p += align256(cells * sizeof(SubStat));
-    auto *maps0 = reinterpret_cast<SubMaps *>(p);
+    auto *maps = reinterpret_cast<SubMaps *>(p);       // of one chain, then of the other
     p += align256(cells * sizeof(SubMaps));
-    auto *maps1 = reinterpret_cast<SubMaps *>(p);
-    p += align256(cells * sizeof(SubMaps));
+    auto *gmaps = reinterpret_cast<SubMaps *>(p);
+    p += align256(cells * kGroups * sizeof(SubMaps));
     auto *rows = reinterpret_cast<RowInfo *>(p);
     const dim3 grid(nsub, batch);
     if (temperature <= 0.0f) {
@@ -531,14 +554,14 @@ int launch_sample(const float *logits, int n, int batch, size_t ld, float temper
     hipLaunchKernelGGL(smp_weights, grid, dim3(kThreads), 0, s, logits, n, ld, inv_t, scale, temperature, w, ldw,
                        stats, rows);
     if (!hip_ok(hipGetLastError(), "sample weights launch")) return -1;
-    hipLaunchKernelGGL(smp_maps, grid, dim3(kThreads), 0, s, w, n, ldw, 0, stats, rows, maps0);
+    hipLaunchKernelGGL(smp_maps, grid, dim3(kThreads), 0, s, w, n, ldw, 0, stats, rows, maps, gmaps);
     if (!hip_ok(hipGetLastError(), "sample maps launch")) return -1;
-    hipLaunchKernelGGL(smp_walk, dim3(batch), dim3(kWave), 0, s, w, n, ldw, 0, nsub, maps0, rows, draws, d_step,
+    hipLaunchKernelGGL(smp_walk, dim3(batch), dim3(kWave), 0, s, w, n, ldw, 0, nsub, maps, gmaps, rows, draws, d_step,
                        batch, tokens);
     if (!hip_ok(hipGetLastError(), "sample sum walk launch")) return -1;
-    hipLaunchKernelGGL(smp_maps, grid, dim3(kThreads), 0, s, w, n, ldw, 1, stats, rows, maps1);
+    hipLaunchKernelGGL(smp_maps, grid, dim3(kThreads), 0, s, w, n, ldw, 1, stats, rows, maps, gmaps);
     if (!hip_ok(hipGetLastError(), "sample maps launch")) return -1;
-    hipLaunchKernelGGL(smp_walk, dim3(batch), dim3(kWave), 0, s, w, n, ldw, 1, nsub, maps1, rows, draws, d_step,
+    hipLaunchKernelGGL(smp_walk, dim3(batch), dim3(kWave), 0, s, w, n, ldw, 1, nsub, maps, gmaps, rows, draws, d_step,
                        batch, tokens);
     return hip_ok(hipGetLastError(), "sample draw walk launch") ? 0 : -1;
 }
