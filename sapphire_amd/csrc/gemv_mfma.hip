@@ -146,38 +146,44 @@ struct TileRegs {
 };
 
 template <int DT, int NG>
-__device__ __forceinline__ void tile_issue(TileRegs<NG> &R, __amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rs,
-                                           int t, int lane) {
+__device__ __forceinline__ void group_issue(TileRegs<NG> &R, __amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rs,
+                                            int t, int g, int lane) {
     constexpr int NQ = DT == DT_Q8_0 ? 2 : 1;
     const int jc = (lane & 15) >> 2, m = lane >> 4;
+    const uint32_t gb = (uint32_t)(t * NG + g);
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        const uint32_t gb = (uint32_t)(t * NG + g);
+    for (int h = 0; h < NQ; ++h) R.a[g][h] = load16(rq, (gb * NQ + h) * 1024u + lane * 16u);
+    R.sv[g] = load16(rs, ((gb * 4u + jc) * 16u + 4u * m) * 4u);
+}
+
+template <int DT, int NG>
+__device__ __forceinline__ void tile_issue(TileRegs<NG> &R, __amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rs,
+                                           int t, int lane) {
 #pragma unroll
-        for (int h = 0; h < NQ; ++h) R.a[g][h] = load16(rq, (gb * NQ + h) * 1024u + lane * 16u);
-        R.sv[g] = load16(rs, ((gb * 4u + jc) * 16u + 4u * m) * 4u);
-    }
+    for (int g = 0; g < NG; ++g) group_issue<DT, NG>(R, rq, rs, t, g, lane);
 }
 
 // Four MFMAs per group (one per block; the lane's B digits enter only the MFMA of the
 // block its column belongs to) and the scales applied to the C values: acc[r] = this
 // lane's column of rows 4m + r.
 template <int DT, int NG>
+__device__ __forceinline__ void group_mfma(const TileRegs<NG> &R, long bop, float p, int g, int lane, float (&acc)[4]) {
+    const int jc = (lane & 15) >> 2;
+    i32x4 C = {0, 0, 0, 0};
+#pragma unroll
+    for (int jj = 0; jj < kGroupBlocks; ++jj)
+        C = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_operand<DT>(R.a[g], jj), jc == jj ? bop : 0L, C, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf((float)C[r], __uint_as_float(R.sv[g][r]) * p, acc[r]);
+}
+
+template <int DT, int NG>
 __device__ __forceinline__ void tile_mfma(const TileRegs<NG> &R, const long (&bop)[NG], const float (&p)[NG],
                                           int lane, float (&acc)[4]) {
-    const int jc = (lane & 15) >> 2;
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[r] = 0.f;
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        i32x4 C = {0, 0, 0, 0};
-#pragma unroll
-        for (int jj = 0; jj < kGroupBlocks; ++jj)
-            C = __builtin_amdgcn_mfma_i32_16x16x32_i8(a_operand<DT>(R.a[g], jj), jc == jj ? bop[g] : 0L, C, 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            acc[r] = __builtin_fmaf((float)C[r], __uint_as_float(R.sv[g][r]) * p[g], acc[r]);
-    }
+    for (int g = 0; g < NG; ++g) group_mfma<DT, NG>(R, bop[g], p[g], g, lane, acc);
 }
 
 // Running (max, sum of exp(v - max), first index of the max) of a stream of logits: the
@@ -286,9 +292,12 @@ __device__ __forceinline__ void tile_store(const float (&acc)[4], float *__restr
 }
 
 // Waves walk the 16-row tiles with a grid stride. Where two tiles' loads fit in registers
-// (DB) the next tile is loaded before the current one is consumed; otherwise its loads
-// are issued as soon as the current tile's MFMAs have read their operands. Each wave
-// builds its B digits once. With kEpSoftmax every workgroup also leaves the softmax/argmax
+// (DB) the next tile is loaded before the current one is consumed; longer rows refill each
+// group's registers from the next tile as soon as its MFMAs have read them, so that one tile of
+// loads stays in flight in one tile of registers and two waves fit a SIMD. (Refilled a whole
+// tile at a time, or two tiles deep, those rows kept one wave per SIMD or waited for every tile.
+// 262144 rows with the softmax: Q4_0 K = 1152 48.8 -> 37.2 us, K = 1024 36.3 -> 33.7; Q8_0 61.1 ->
+// 56.2 and 56.1 -> 51.9. Three waves per SIMD instead of two spill and measured slower.) Each wave builds its B digits once. With kEpSoftmax every workgroup also leaves the softmax/argmax
 // partial of its rows in part[blockIdx.x] (folded by softmax_finish_parts). With
 // kEpGreedyStep every workgroup leaves the greedy key of its rows in its slot of gs.keys and
 // counts itself done; the last one takes the maximum key, decodes the token and advances the
@@ -297,12 +306,11 @@ __device__ __forceinline__ void tile_store(const float (&acc)[4], float *__restr
 // the step (gs.slots->b), and workgroup 0 writes gs.slots->a = b: the next step's layers
 // kernel picks the token.
 template <int DT, int NG, int EP>
-__global__ __launch_bounds__(256) void gemv_mfma(const uint8_t *__restrict__ wq, uint32_t q_bytes,
+__global__ __launch_bounds__(256, NG > 5 ? 2 : 1) void gemv_mfma(const uint8_t *__restrict__ wq, uint32_t q_bytes,
                                                  const uint8_t *__restrict__ wsc, uint32_t s_bytes,
                                                  const float *__restrict__ x, float *__restrict__ y, int M,
                                                  int ntiles, SoftPart *__restrict__ part, GreedyStep gs) {
-    constexpr int NQ = DT == DT_Q8_0 ? 2 : 1;
-    constexpr bool DB = NG * (NQ + 1) * 4 * 2 <= 128;   // VGPRs of two tiles' loads
+    constexpr bool DB = NG <= 5;
     const int lane = threadIdx.x & (kWave - 1), nw_blk = blockDim.x / kWave;
     const int wave = blockIdx.x * nw_blk + threadIdx.x / kWave;
     const int nwaves = gridDim.x * nw_blk;
@@ -349,11 +357,22 @@ __global__ __launch_bounds__(256) void gemv_mfma(const uint8_t *__restrict__ wq,
         }
     } else {
         while (t < ntiles) {
-            tile_mfma<DT, NG>(RA, bop, p, lane, acc);
-            const int tn = t + nwaves;
-            if (tn < ntiles) tile_issue<DT, NG>(RA, rq, rs, tn, lane);
+            // past the last tile the refills repeat it: the loads in flight, and so the waits,
+            // are the same in every trip
+            const int tn = min(t + nwaves, ntiles - 1);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[r] = 0.f;
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                // the four masked forms of a group's digits are made here, not kept (8 NG registers)
+                asm volatile("" : "+v"(bop[g]));
+                group_mfma<DT, NG>(RA, bop[g], p[g], g, lane, acc);
+                asm volatile("" ::: "memory");
+                group_issue<DT, NG>(RA, rq, rs, tn, g, lane);
+                asm volatile("" ::: "memory");
+            }
             tile_store<DT, EP>(acc, y, M, t, lane, sp, key, nc);
-            t = tn;
+            t += nwaves;
         }
     }
     if constexpr (EP == kEpGreedyStep) {
@@ -584,14 +603,18 @@ int cus_of_current_device() {
 // Waves per CU of the TILED GEMV. Measured on the 262144 x 640 LM head with cold weights:
 // Q8_0 (11.5 KiB per tile) is fastest at 8 (two per SIMD, its register limit for the double
 // buffer anyway), Q4_0 (6.4 KiB per tile, half the bytes per wave) at 12 (3 %).
-constexpr int kWavesPerCuQ8 = 8, kWavesPerCuQ4 = 12;
+// Rows of more than five groups are bound to two waves per SIMD by their registers.
+constexpr int kWavesPerCu = 8, kWavesPerCuShortQ4 = 12;
 
-unsigned tiled_blocks(int dt, int M) {
+unsigned tiled_blocks(int dt, int M, int K) {
     const int ntiles = (M + kTileRows - 1) / kTileRows;
-    const int per_cu = dt == DT_Q4_0 ? kWavesPerCuQ4 : kWavesPerCuQ8;
+    const int per_cu = dt == DT_Q4_0 && K <= 5 * kGroupBlocks * kBlock ? kWavesPerCuShortQ4 : kWavesPerCu;
     const long waves = std::min<long>(ntiles, (long)cus_of_current_device() * per_cu);
     return (unsigned)((waves + 3) / 4);
 }
+
+// the most workgroups of any dtype and row length
+size_t tiled_max_blocks(int M) { return tiled_blocks(DT_Q4_0, M, 0); }
 
 template <int DT, int NG>
 int launch_mfma_typed(const uint8_t *w, int M, int K, const float *x, float *y, SoftPart *part,
@@ -599,7 +622,7 @@ int launch_mfma_typed(const uint8_t *w, int M, int K, const float *x, float *y, 
     const int ntiles = (M + kTileRows - 1) / kTileRows;
     const size_t so = q_tiled_scales_offset(DT, M, K);
     const size_t sbytes = q_tiled_bytes(DT, M, K) - so;
-    const unsigned blocks = tiled_blocks(DT, M);
+    const unsigned blocks = tiled_blocks(DT, M, K);
     const GreedyStep g = gs ? *gs : GreedyStep{};
     if (gs && gs->slots)
         hipLaunchKernelGGL((gemv_mfma<DT, NG, kEpGreedySlots>), dim3(blocks), dim3(256), 0, st, w, (uint32_t)so,
@@ -680,7 +703,7 @@ int launch_tiled_unpack(int dt, const void *w, int M, int K, int8_t *ints, float
 }
 
 size_t tiled_softmax_scratch_bytes(int M) {
-    return sizeof(SoftPart) * (size_t)std::max(tiled_blocks(DT_Q4_0, M), tiled_blocks(DT_Q8_0, M));
+    return sizeof(SoftPart) * tiled_max_blocks(M);
 }
 
 int launch_gemv_tiled_softmax(int dt, const void *w, int M, int K, const float *x, float *logits, float *probs,
@@ -695,7 +718,7 @@ int launch_gemv_tiled_softmax(int dt, const void *w, int M, int K, const float *
     const int chunk = ((M + blocks - 1) / blocks + 3) & ~3;
     const int aligned = ((reinterpret_cast<uintptr_t>(logits) | reinterpret_cast<uintptr_t>(probs)) & 15u) == 0;
     hipLaunchKernelGGL(softmax_finish_parts, dim3(blocks), dim3(256), 0, st, logits, M, chunk, part,
-                       (int)tiled_blocks(dt, M), probs, argmax, aligned);
+                       (int)tiled_blocks(dt, M, K), probs, argmax, aligned);
     return hip_ok(hipGetLastError(), "softmax_finish_parts launch") ? 0 : -1;
 }
 
@@ -703,7 +726,7 @@ int launch_gemv_tiled(int dt, const void *w, int M, int K, const float *x, float
     return launch_tiled(dt, w, M, K, x, y, nullptr, st);
 }
 
-size_t tiled_greedy_key_slots(int M) { return std::max(tiled_blocks(DT_Q4_0, M), tiled_blocks(DT_Q8_0, M)); }
+size_t tiled_greedy_key_slots(int M) { return tiled_max_blocks(M); }
 
 int launch_gemv_tiled_greedy_step(int dt, const void *w, int M, int K, const float *x, float *logits,
                                   const GreedyStep &gs, hipStream_t st) {
