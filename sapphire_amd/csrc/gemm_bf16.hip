@@ -1,4 +1,4 @@
-// gemm_bf16.hip - BF16 weights times a batch of up to 16 fp32 activation vectors on the CDNA4
+// gemm_bf16.hip - BF16 weights times a batch of up to 32 fp32 activation vectors on the CDNA4
 // matrix cores: Y[b][r] = sum_k W[r][k] * X[b][k], the batched form of kernel_gemv for BF16
 // tensors (kernel_gemv_batch / kernel_gemm, dispatch.c:87-99,234-266; the reference computes it
 // with kernel_gemm_bf16_avx2, bf16_avx.c:115-159).
@@ -12,10 +12,12 @@
 //    bf16 has fp32's exponent range, so no range scaling is needed.
 //  * C: per lane the four sequences 4m..4m+3 (m = l / 16) of weight row l % 16, accumulated
 //    over the blocks in order, three terms per block.
-// A workgroup of four waves stages a 256-element chunk of all 16 vectors' terms into LDS
-// (24 KiB) and each wave multiplies its tiles (grid-stride, at most kMaxTiles per wave, their
-// accumulators held across the chunks). The weight loads of a tile's eight blocks are issued
+// A workgroup of four waves stages the terms of a chunk of K (256 elements of 16 vectors, or 128
+// of 32: 24 KiB) into LDS and each wave multiplies its tiles (grid-stride, at most kMaxTiles per
+// wave, their accumulators held across the chunks). The weight loads of a tile's chunk are issued
 // together, up to three tiles ahead of the one being multiplied (across chunk boundaries too).
+// 17 to 32 vectors share one pass over the weights, their terms held in registers (262144 x 640:
+// 17 vectors 135 us in two passes, 73 us in one; 32 vectors 146 and 90 us).
 #include <algorithm>
 
 #include "internal.h"
@@ -28,11 +30,10 @@ constexpr int kWave = 64;
 constexpr int kWavesPerWg = 4;
 constexpr int kThreads = kWave * kWavesPerWg;
 constexpr int kTileRows = 16;
-constexpr int kChunk = 256;                 // elements of K staged at a time
-constexpr int kChunkBlocks = kChunk / 32;
+constexpr int kStageBlocks = 8;             // (token tile, block) pairs staged at a time
 constexpr int kTerms = 3;
 constexpr int kMaxTiles = 8;                // tiles per wave (accumulators in registers)
-constexpr int kBatch = 16;
+constexpr int kSeqs = 16;                   // vectors of a token tile
 constexpr uint32_t kOffNone = 0xFFFFFFF0u;  // out of range: the buffer load returns zeros
 constexpr int kNT = 0;                      // plain loads: a row's two 64-byte halves meet in L2
 
@@ -51,11 +52,12 @@ __device__ __forceinline__ uint32_t bf16_rne(float x) {
 }
 __device__ __forceinline__ float bf16_to_f(uint32_t b) { return __uint_as_float(b << 16); }
 
-template <int NTW>
+template <int NTW, int NTT>
 __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const uint16_t *__restrict__ w, uint32_t w_bytes, int M,
-                                                             int K, const float *__restrict__ x, int ldx, int batch,
-                                                             float *__restrict__ y, int ldy) {
-    __shared__ u32x4 as[kTerms][kChunkBlocks][kWave];   // the A operands of a chunk (24 KiB)
+                                                                int K, const float *__restrict__ x, int ldx, int batch,
+                                                                float *__restrict__ y, int ldy) {
+    constexpr int kChunkBlocks = kStageBlocks / NTT, kChunk = kChunkBlocks * 32;
+    __shared__ u32x4 as[kTerms][NTT][kChunkBlocks][kWave];   // the A operands of a chunk (24 KiB)
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid / kWave;
     const int n = lane & 15, m = lane >> 4;
     const int ntiles = (M + kTileRows - 1) / kTileRows;
@@ -64,9 +66,11 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const uint16_t *__r
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(w, w_bytes);
     const uint32_t row_bytes = (uint32_t)K * 2u;
 
-    f4 acc[NTW];
+    f4 acc[NTW][NTT];
 #pragma unroll
-    for (int i = 0; i < NTW; ++i) acc[i] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NTW; ++i)
+#pragma unroll
+        for (int q = 0; q < NTT; ++q) acc[i][q] = f4{0.f, 0.f, 0.f, 0.f};
 
     // A ring of R tile loads: unit u = (chunk, tile i) sits in bw[u % R] = bw[i % R] (NTW is a
     // multiple of R), and unit u + R - 1 is issued while unit u is multiplied, across chunk
@@ -87,14 +91,15 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const uint16_t *__r
 #pragma unroll
     for (int j = 0; j + 1 < R; ++j) issue(0, j, bw[j]);   // in flight during the first staging
     for (int k0 = 0; k0 < K; k0 += kChunk) {
-        // ---- stage: thread (seq, q) converts elements k0 + 16q .. + 15 of vector seq ----
+        // ---- stage: thread (seq, q) converts elements 16 q .. + 15 of the chunk of vector seq ----
         {
-            const int seq = tid & 15, q = tid >> 4;
-            const int bl = q >> 1;
+            const int seq = tid & 15, pair = tid >> 5;   // 8 (token tile, block) pairs
+            const int tt0 = pair / kChunkBlocks, bl = pair % kChunkBlocks;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int g = (q & 1) * 2 + h;                  // 8-element group of the block
+                const int g = (tid >> 4 & 1) * 2 + h;           // 8-element group of the block
                 const int kk = k0 + bl * 32 + g * 8;
+                const int vec = tt0 * kSeqs + seq;
                 uint32_t t[kTerms][4];
 #pragma unroll
                 for (int e = 0; e < 8; e += 2) {
@@ -102,7 +107,7 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const uint16_t *__r
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         const int k = kk + e + u;
-                        v[u] = (seq < batch && k < K) ? x[(size_t)seq * ldx + k] : 0.f;
+                        v[u] = (vec < batch && k < K) ? x[(size_t)vec * ldx + k] : 0.f;
                     }
                     uint32_t b[kTerms][2];
 #pragma unroll
@@ -118,12 +123,24 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const uint16_t *__r
                 }
 #pragma unroll
                 for (int tt = 0; tt < kTerms; ++tt)
-                    as[tt][bl][g * 16 + seq] = u32x4{t[tt][0], t[tt][1], t[tt][2], t[tt][3]};
+                    as[tt][tt0][bl][g * 16 + seq] = u32x4{t[tt][0], t[tt][1], t[tt][2], t[tt][3]};
             }
         }
         __syncthreads();
+        // two token tiles: the operands go to registers, and LDS is free for the next staging
+        constexpr bool kHeld = NTT > 1;
+        u32x4 a[NTT][kChunkBlocks][kTerms];
+        if constexpr (kHeld) {
+#pragma unroll
+            for (int q = 0; q < NTT; ++q)
+#pragma unroll
+                for (int b = 0; b < kChunkBlocks; ++b)
+#pragma unroll
+                    for (int tt = 0; tt < kTerms; ++tt) a[q][b][tt] = as[tt][q][b][lane];
+            __syncthreads();
+        }
         const int nbl = min(kChunkBlocks, (K - k0 + 31) / 32);
-        // ---- multiply the wave's tiles ----
+        // ---- multiply the wave's tiles (blocks past K are zeros on both sides) ----
 #pragma unroll
         for (int i = 0; i < NTW; ++i) {
             const int ia = i + R - 1;   // the unit issued now: R - 1 ahead
@@ -136,13 +153,15 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const uint16_t *__r
                         const bf16x8 bop = __builtin_bit_cast(bf16x8, bw[i % R][b]);
 #pragma unroll
                         for (int tt = 0; tt < kTerms; ++tt)
-                            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                __builtin_bit_cast(bf16x8, as[tt][b][lane]), bop, acc[i], 0, 0, 0);
+#pragma unroll
+                            for (int q = 0; q < NTT; ++q)
+                                acc[i][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    __builtin_bit_cast(bf16x8, kHeld ? a[q][b][tt] : as[tt][q][b][lane]), bop, acc[i][q], 0, 0, 0);
                     }
                 }
             }
         }
-        __syncthreads();   // the chunk's A operands are read before the next staging
+        if constexpr (!kHeld) __syncthreads();   // the operands are read before the next staging
     }
 #pragma unroll
     for (int i = 0; i < NTW; ++i) {
@@ -150,8 +169,12 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const uint16_t *__r
         const int row = t * kTileRows + n;
         if (t < ntiles && row < M)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (4 * m + r < batch) y[(size_t)(4 * m + r) * ldy + row] = acc[i][r];
+            for (int q = 0; q < NTT; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int vec = q * kSeqs + 4 * m + r;
+                    if (vec < batch) y[(size_t)vec * ldy + row] = acc[i][q][r];
+                }
     }
 }
 
@@ -179,8 +202,9 @@ int launch_gemm_bf16(const void *w, int M, int K, const float *x, int ldx, int b
     static const int cus = cus_bf16();
     const long ntiles = (M + kTileRows - 1) / kTileRows;
     const uint32_t wb = (uint32_t)((size_t)M * K * 2);
-    for (int b0 = 0; b0 < batch; b0 += kBatch) {
-        const int nb = std::min(kBatch, batch - b0);
+    const int pass = batch > kSeqs ? 2 * kSeqs : kSeqs;
+    for (int b0 = 0; b0 < batch; b0 += pass) {
+        const int nb = std::min(pass, batch - b0);
         // waves: up to eight per CU, enough that no wave has more than kMaxTiles tiles
         const long waves = std::max(std::min(ntiles, 8L * cus), (ntiles + kMaxTiles - 1) / kMaxTiles);
         const int ntw = (int)((ntiles + waves - 1) / waves);
@@ -188,13 +212,12 @@ int launch_gemm_bf16(const void *w, int M, int K, const float *x, int ldx, int b
         const float *xb = x + (size_t)b0 * ldx;
         float *yb = y + (size_t)b0 * ldy;
         const uint16_t *wp = static_cast<const uint16_t *>(w);
-        switch (ntw) {
-            case 1: hipLaunchKernelGGL(gemm_bf16_kernel<1>, grid, blk, 0, st, wp, wb, M, K, xb, ldx, nb, yb, ldy); break;
-            case 2: hipLaunchKernelGGL(gemm_bf16_kernel<2>, grid, blk, 0, st, wp, wb, M, K, xb, ldx, nb, yb, ldy); break;
-            case 3:
-            case 4: hipLaunchKernelGGL(gemm_bf16_kernel<4>, grid, blk, 0, st, wp, wb, M, K, xb, ldx, nb, yb, ldy); break;
-            default: hipLaunchKernelGGL(gemm_bf16_kernel<8>, grid, blk, 0, st, wp, wb, M, K, xb, ldx, nb, yb, ldy); break;
-        }
+        auto pick = [&](auto one, auto two) { return nb > kSeqs ? two : one; };
+        auto kern = ntw == 1   ? pick(gemm_bf16_kernel<1, 1>, gemm_bf16_kernel<1, 2>)
+                    : ntw == 2 ? pick(gemm_bf16_kernel<2, 1>, gemm_bf16_kernel<2, 2>)
+                    : ntw <= 4 ? pick(gemm_bf16_kernel<4, 1>, gemm_bf16_kernel<4, 2>)
+                               : pick(gemm_bf16_kernel<8, 1>, gemm_bf16_kernel<8, 2>);
+        hipLaunchKernelGGL(kern, grid, blk, 0, st, wp, wb, M, K, xb, ldx, nb, yb, ldy);
         if (!hip_ok(hipGetLastError(), "gemm_bf16 launch")) return -1;
     }
     return 0;

@@ -60,3 +60,20 @@ def test_gemm_wide_non_finite(hip, oracle, dtype, m, k):
     ref = _ref(oracle, dtype, W, X)
     for b in range(40):
         _same_special(got[b], ref[b])
+
+
+@pytest.mark.parametrize("m,k,batch", [(300, 96, 17), (16, 136, 32), (2048, 640, 33), (40000, 264, 31), (150000, 128, 48)],
+                         ids=lambda v: str(v))
+def test_gemm_bf16_two_token_tiles(hip, m, k, batch):
+    """17 to 32 vectors in one pass over BF16 weights (K remainders of a 128-element chunk, every
+    number of tiles per wave, a last pass of one tile). Products are exact in three terms, so the
+    bound is the fp32 sum's: 2 sqrt(3 K) 2^-24 of sum |w x|, and one vector's bits do not depend on
+    how many share the pass."""
+    from tests.test_gemv_f_gpu import run_gemm_bf16
+    W = synth.bf16_normal((m, k), 54, m)
+    X = synth.normal_f32((batch, k), 54, 2)
+    got = run_gemm_bf16(W, X)
+    w = (W.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    ref, mag = X.astype(np.float64) @ w.T, np.abs(X.astype(np.float64)) @ np.abs(w).T
+    assert np.all(np.abs(got - ref) <= 2.0 * np.sqrt(3 * k) * 2.0 ** -24 * mag)
+    assert np.array_equal(run_gemm_bf16(W, X[:5]), got[:5])
