@@ -14,8 +14,17 @@
 // divisions are correctly rounded. Inputs must be finite; a block whose scale is subnormal
 // (1/d overflows) saturates infinite products and codes NaN ones (0 * inf) as zero.
 //
+// The codes are a few operations per element: the block's largest and smallest value give its
+// maximum and (Q4_0) the sign of the first element that has it, unless both signs do; roundings
+// are conversions, their saturation covering the clamps. What those forms get wrong (a NaN or
+// infinite element, a scale whose reciprocal overflows) goes through the plain ones, a wave at a
+// time. Before, with the index of the first maximum tracked and every code clamped by compares,
+// the arithmetic alone took about as long as the memory (262144 x 640 BF16 to Q4_0 110 us, now 98;
+// 262144 x 1151, rows starting anywhere, 349 us with single-element loads, now 177).
+//
 // Layout of the work: four lanes per block, lane l holding elements 8l..8l+7 (two 16-byte
-// fp32 loads or one 16-byte bf16 load, consecutive lanes on consecutive bytes); the block's
+// fp32 loads or one 16-byte bf16 load, consecutive lanes on consecutive bytes; rows that start
+// anywhere by the same loads, unaligned); the block's
 // maximum goes through two DPP steps inside the quad. A Q4_0 lane stores one dword of
 // nibbles, a Q8_0 lane two dwords of quants, lane 0 the scale (plain stores, so the L2
 // merges a wave's partial lines before they go to HBM). Each lane group loads 128
@@ -44,6 +53,10 @@ __device__ __forceinline__ float max4(float v) {
     v = fmaxf(v, lanes::dpp_mov<0xB1>(v));
     return fmaxf(v, lanes::dpp_mov<0x4E>(v));
 }
+__device__ __forceinline__ float min4(float v) {
+    v = fminf(v, lanes::dpp_mov<0xB1>(v));
+    return fminf(v, lanes::dpp_mov<0x4E>(v));
+}
 __device__ __forceinline__ int min4(int v) {
     v = min(v, dpp_int<0xB1>(v));
     return min(v, dpp_int<0x4E>(v));
@@ -57,23 +70,36 @@ __device__ __forceinline__ int q8_code(float v) {
 }
 __device__ __forceinline__ int q4_code(float v) { return v != v ? 8 : v > 15.0f ? 15 : v < 0.0f ? 0 : (int)v; }
 
-// Elements e0..e0+7 of a row (zeros past K), without branches: VEC (K % 8 == 0, 16-byte
-// aligned rows) loads the eight at a clamped address and zeroes them past the row; otherwise
-// each element is loaded from a clamped index and zeroed past the row.
-template <int SRC, bool VEC>
+// How a lane reads its eight elements: 16-byte aligned (K % 8 == 0 and an aligned source), at any
+// alignment (K >= 8), or one by one.
+enum Access { kAligned = 0, kUnaligned = 1, kSingle = 2 };
+
+// Elements e0..e0+7 of a row (zeros past K), without branches around the loads: the eight are
+// loaded at an address clamped into the row and zeroed (kUnaligned: shifted into place) past it.
+template <int SRC, int ACC>
 __device__ __forceinline__ void load8(const void *__restrict__ src, size_t base, int e0, int K, float (&x)[8]) {
     const bool in = e0 < K;
-    if constexpr (VEC) {
-        const size_t off = base + (in ? e0 : 0);
+    if constexpr (ACC != kSingle) {
+        const int at = ACC == kAligned ? (in ? e0 : 0) : min(e0, K - 8);
+        const size_t off = base + at;
         float v[8];
         if constexpr (SRC == DT_F32) {
-            const f32x4 *p = reinterpret_cast<const f32x4 *>(static_cast<const float *>(src) + off);
-            const f32x4 a = __builtin_nontemporal_load(p), b = __builtin_nontemporal_load(p + 1);
+            const float *p = static_cast<const float *>(src) + off;
+            f32x4 a, b;
+            if constexpr (ACC == kAligned) {
+                a = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p));
+                b = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p) + 1);
+            } else {
+                __builtin_memcpy(&a, p, 16);
+                __builtin_memcpy(&b, p + 4, 16);
+            }
             v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
             v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
         } else {
-            const u32x4 t =
-                __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(src) + off));
+            const uint16_t *p = static_cast<const uint16_t *>(src) + off;
+            u32x4 t;
+            if constexpr (ACC == kAligned) t = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+            else __builtin_memcpy(&t, p, 16);
             const uint32_t w[4] = {t.x, t.y, t.z, t.w};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -81,8 +107,13 @@ __device__ __forceinline__ void load8(const void *__restrict__ src, size_t base,
                 v[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
             }
         }
+        if constexpr (ACC == kAligned) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = in ? v[i] : 0.f;
+            for (int i = 0; i < 8; ++i) x[i] = in ? v[i] : 0.f;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[i] = v[i];
+        }
     } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -96,9 +127,26 @@ __device__ __forceinline__ void load8(const void *__restrict__ src, size_t base,
     }
 }
 
+// kUnaligned: the eight elements loaded at min(e0, K - 8) moved down by what was clamped (8 and
+// more: all zeros), for the lanes at a row's end.
+__device__ __forceinline__ void shift_into_place(int e0, int K, float (&x)[8]) {
+    const int sh = e0 - min(e0, K - 8);
+    if (!__any(sh != 0)) return;
+#pragma unroll
+    for (int bit = 4; bit >= 1; bit >>= 1)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = (sh & bit) ? (i + bit < 8 ? x[i + bit] : 0.f) : x[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = sh >= 8 ? 0.f : x[i];
+}
+
+// roundf(v) as an integer for |v| < 2^22: adding the float below 1/2 towards v's sign and
+// truncating rounds halves away from zero and everything else to the nearest.
+__device__ __forceinline__ int round_away(float v) { return (int)__fadd_rn(v, copysignf(0x1.fffffep-2f, v)); }
+
 // DENSE: K % 32 == 0, so block b starts at element 32b. Otherwise row and block come from a
 // 32-bit division (the launcher keeps such matrices below 2^31 blocks).
-template <int DST, int SRC, bool VEC, bool DENSE, int U>
+template <int DST, int SRC, int ACC, bool DENSE, int U>
 __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restrict__ src, int K, int nb,
                                                             long nblocks, uint8_t *__restrict__ dst) {
     constexpr int BB = DST == DT_Q4_0 ? 20 : 36;
@@ -112,11 +160,11 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restr
         for (int u = 0; u < U; ++u) {
             const long b = min(b0 + u * stride, nblocks - 1);
             if constexpr (DENSE) {
-                load8<SRC, VEC>(src, (size_t)b * 32, lq * 8, 32, x[u]);
+                load8<SRC, ACC>(src, (size_t)b * 32, lq * 8, 32, x[u]);
             } else {
                 const uint32_t row = (uint32_t)b / (uint32_t)nb;
                 const int blk = (int)((uint32_t)b - row * (uint32_t)nb);
-                load8<SRC, VEC>(src, (size_t)row * K, blk * 32 + lq * 8, K, x[u]);
+                load8<SRC, ACC>(src, (size_t)row * K, blk * 32 + lq * 8, K, x[u]);
             }
         }
 #pragma unroll
@@ -124,25 +172,59 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restr
             const long b = b0 + u * stride;
             const bool store = b < nblocks;   // the same for the four lanes of a block
             uint8_t *out = dst + (size_t)min(b, nblocks - 1) * BB;
-            float la = 0.f;
-            int lkey = 0x7FFFFFFF;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float a = fabsf(x[u][i]);
-                const bool gt = la < a;   // the first element of the lane's largest |x|
-                la = gt ? a : la;
-                if constexpr (DST == DT_Q4_0)
-                    lkey = gt ? (((lq * 8 + i) << 1) | (int)(__float_as_uint(x[u][i]) >> 31)) : lkey;
+            if constexpr (ACC == kUnaligned) {
+                // the row's elements sit in row order in the row's blocks
+                const uint32_t bb = (uint32_t)min(b, nblocks - 1);
+                if constexpr (!DENSE) shift_into_place((int)(bb % (uint32_t)nb) * 32 + lq * 8, K, x[u]);
             }
-            const float amax = max4(la);
-            if constexpr (DST == DT_Q8_0) {
-                const float d = amax / 127.0f;
-                const float id = d != 0.f ? 1.0f / d : 0.f;
-                uint32_t w[2] = {0u, 0u};
+            float top = x[u][0], low = x[u][0];
+            bool nan = false;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int q = q8_code(roundf(__fmul_rn(x[u][i], id)));
-                    w[i >> 2] |= (uint32_t)(q & 0xFF) << (8 * (i & 3));
+            for (int i = 1; i < 8; ++i) {
+                top = fmaxf(top, x[u][i]);
+                low = fminf(low, x[u][i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) nan |= __builtin_isunordered(x[u][i], x[u][i + 1]);
+            top = max4(top);
+            low = min4(low);
+            const float amax = fmaxf(fmaxf(top, -low), 0.f);   // NaN elements never count
+            float d, id;
+            if constexpr (DST == DT_Q8_0) {
+                d = amax / 127.0f;
+                id = d != 0.f ? 1.0f / d : 0.f;
+            } else {
+                float mx = top > -low ? amax : -amax;
+                // both signs reach the maximum: the first element (in block order) that does
+                if (__any(top == -low)) {
+                    int key = 0x7FFFFFFF;
+#pragma unroll
+                    for (int i = 7; i >= 0; --i)
+                        key = fabsf(x[u][i]) == amax ? ((lq * 8 + i) << 1) | (int)(__float_as_uint(x[u][i]) >> 31) : key;
+                    key = min4(key);
+                    mx = top == -low ? ((key & 1) ? -amax : amax) : mx;
+                }
+                mx = amax == 0.f ? 0.f : mx;
+                d = mx / -8.0f;
+                id = d != 0.f ? 1.0f / d : 0.f;
+            }
+            // |id| overflows or the maximum is infinite (then id is 0): infinite and NaN products
+            const bool plain = __any(nan || !(amax < INFINITY) || !(fabsf(id) < INFINITY)) != 0;
+            if constexpr (DST == DT_Q8_0) {
+                uint32_t w[2] = {0u, 0u};
+                if (!plain) {
+#pragma unroll
+                    for (int i = 0; i < 8; i += 4) {
+                        uint32_t q[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) q[e] = (uint32_t)round_away(__fmul_rn(x[u][i + e], id));
+                        w[i >> 2] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(q[3], q[2], 0x0C0C0400u),
+                                                          __builtin_amdgcn_perm(q[1], q[0], 0x0C0C0400u), 0x05040100u);
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        w[i >> 2] |= (uint32_t)(q8_code(roundf(__fmul_rn(x[u][i], id))) & 0xFF) << (8 * (i & 3));
                 }
                 if (store) {
                     uint32_t *o = reinterpret_cast<uint32_t *>(out + 4) + 2 * lq;
@@ -151,15 +233,17 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restr
                     if (lq == 0) *reinterpret_cast<float *>(out) = d;
                 }
             } else {
-                // the first element (in block order) whose |x| is the block's maximum, and its sign
-                const int key = min4(la == amax ? lkey : 0x7FFFFFFF);
-                const float mx = amax == 0.f ? 0.f : ((key & 1) ? -amax : amax);
-                const float d = mx / -8.0f;
-                const float id = d != 0.f ? 1.0f / d : 0.f;
                 uint32_t w = 0;
+                if (!plain) {
+                    // every value is at least 0.5: only the upper clamp is left
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    w |= (uint32_t)q4_code(__fadd_rn(__fmul_rn(x[u][i], id), 8.5f)) << (4 * i);
+                    for (int i = 0; i < 8; ++i)
+                        w |= min((uint32_t)__fadd_rn(__fmul_rn(x[u][i], id), 8.5f), 15u) << (4 * i);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        w |= (uint32_t)q4_code(__fadd_rn(__fmul_rn(x[u][i], id), 8.5f)) << (4 * i);
+                }
                 if (store) {
                     reinterpret_cast<uint32_t *>(out + 4)[lq] = w;
                     if (lq == 0) *reinterpret_cast<float *>(out) = d;
@@ -193,13 +277,15 @@ int launch_typed(const void *src, int M, int K, void *dst, hipStream_t st) {
     uint8_t *d = static_cast<uint8_t *>(dst);
     const dim3 g((unsigned)grid), t(kQThreads);
     if (vec && K % 32 == 0)
-        hipLaunchKernelGGL((quantize_kernel<DST, SRC, true, true, U>), g, t, 0, st, src, K, nb, nblocks, d);
+        hipLaunchKernelGGL((quantize_kernel<DST, SRC, kAligned, true, U>), g, t, 0, st, src, K, nb, nblocks, d);
     else if (vec)
-        hipLaunchKernelGGL((quantize_kernel<DST, SRC, true, false, U>), g, t, 0, st, src, K, nb, nblocks, d);
+        hipLaunchKernelGGL((quantize_kernel<DST, SRC, kAligned, false, U>), g, t, 0, st, src, K, nb, nblocks, d);
     else if (K % 32 == 0)
-        hipLaunchKernelGGL((quantize_kernel<DST, SRC, false, true, U>), g, t, 0, st, src, K, nb, nblocks, d);
+        hipLaunchKernelGGL((quantize_kernel<DST, SRC, kUnaligned, true, U>), g, t, 0, st, src, K, nb, nblocks, d);
+    else if (K >= 8)
+        hipLaunchKernelGGL((quantize_kernel<DST, SRC, kUnaligned, false, U>), g, t, 0, st, src, K, nb, nblocks, d);
     else
-        hipLaunchKernelGGL((quantize_kernel<DST, SRC, false, false, U>), g, t, 0, st, src, K, nb, nblocks, d);
+        hipLaunchKernelGGL((quantize_kernel<DST, SRC, kSingle, false, U>), g, t, 0, st, src, K, nb, nblocks, d);
     return 0;
 }
 
