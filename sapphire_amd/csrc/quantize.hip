@@ -20,15 +20,16 @@
 // infinite element, a scale whose reciprocal overflows) goes through the plain ones, a wave at a
 // time. Before, with the index of the first maximum tracked and every code clamped by compares,
 // the arithmetic alone took about as long as the memory (262144 x 640 BF16 to Q4_0 110 us, now 98;
-// 262144 x 1151, rows starting anywhere, 349 us with single-element loads, now 177).
+// 262144 x 1151, rows starting anywhere, 349 us with single-element loads, now 177). With the bytes
+// stored through LDS instead of a dword per lane they take 90 and 155 us, 4.9-5.1 TB/s, the rate of
+// a device copy.
 //
 // Layout of the work: four lanes per block, lane l holding elements 8l..8l+7 (two 16-byte
 // fp32 loads or one 16-byte bf16 load, consecutive lanes on consecutive bytes; rows that start
 // anywhere by the same loads, unaligned); the block's
-// maximum goes through two DPP steps inside the quad. A Q4_0 lane stores one dword of
-// nibbles, a Q8_0 lane two dwords of quants, lane 0 the scale (plain stores, so the L2
-// merges a wave's partial lines before they go to HBM). Each lane group loads 128
-// bytes of source (4 fp32 or 8 bf16 blocks) before it quantizes any of them.
+// maximum goes through two DPP steps inside the quad. Each lane loads 64 or 128 bytes of source
+// (4 fp32 or 8 bf16 blocks) before it quantizes any of them; a wave's blocks are consecutive, and
+// their bytes go out through LDS, 16 per lane.
 #include <algorithm>
 
 #include "internal.h"
@@ -38,7 +39,7 @@ namespace sapphire {
 
 namespace {
 
-constexpr int kQThreads = 256;
+constexpr int kQThreads = 256, kWave = 64;
 constexpr int kLanes = 4;   // lanes per block, eight elements each
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -150,15 +151,21 @@ template <int DST, int SRC, int ACC, bool DENSE, int U>
 __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restrict__ src, int K, int nb,
                                                             long nblocks, uint8_t *__restrict__ dst) {
     constexpr int BB = DST == DT_Q4_0 ? 20 : 36;
-    const int lq = threadIdx.x & (kLanes - 1);
-    const long group = ((long)blockIdx.x * kQThreads + threadIdx.x) / kLanes;
-    const long stride = ((long)gridDim.x * kQThreads) / kLanes;
-    for (long b0 = group; b0 < nblocks; b0 += U * stride) {
+    constexpr int kRun = U * kWave / kLanes;           // consecutive blocks of a wave's trip
+    constexpr int kWords = kRun * BB / 4;
+    __shared__ __attribute__((aligned(16))) uint32_t stage[kQThreads / kWave][kWords];
+    const int lq = threadIdx.x & (kLanes - 1), lane = threadIdx.x & (kWave - 1);
+    uint32_t *mine = stage[threadIdx.x / kWave];
+    const long wave = ((long)blockIdx.x * kQThreads + threadIdx.x) / kWave;
+    const long stride = (long)gridDim.x * (kQThreads / kWave) * kRun;
+    const bool wide = (reinterpret_cast<uintptr_t>(dst) & 15) == 0;   // runs are multiples of 16 bytes
+    for (long r0 = wave * kRun; r0 < nblocks; r0 += stride) {
+        const long b0 = r0 + lane / kLanes;
         // every lane loads U blocks (past the end: the last block again), then quantizes them
         float x[U][8];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const long b = min(b0 + u * stride, nblocks - 1);
+            const long b = min(b0 + u * (kWave / kLanes), nblocks - 1);
             if constexpr (DENSE) {
                 load8<SRC, ACC>(src, (size_t)b * 32, lq * 8, 32, x[u]);
             } else {
@@ -169,9 +176,8 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restr
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const long b = b0 + u * stride;
-            const bool store = b < nblocks;   // the same for the four lanes of a block
-            uint8_t *out = dst + (size_t)min(b, nblocks - 1) * BB;
+            const long b = b0 + u * (kWave / kLanes);
+            uint32_t *out = mine + (u * (kWave / kLanes) + lane / kLanes) * (BB / 4);
             if constexpr (ACC == kUnaligned) {
                 // the row's elements sit in row order in the row's blocks
                 const uint32_t bb = (uint32_t)min(b, nblocks - 1);
@@ -226,12 +232,8 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restr
                     for (int i = 0; i < 8; ++i)
                         w[i >> 2] |= (uint32_t)(q8_code(roundf(__fmul_rn(x[u][i], id))) & 0xFF) << (8 * (i & 3));
                 }
-                if (store) {
-                    uint32_t *o = reinterpret_cast<uint32_t *>(out + 4) + 2 * lq;
-                    o[0] = w[0];
-                    o[1] = w[1];
-                    if (lq == 0) *reinterpret_cast<float *>(out) = d;
-                }
+                out[1 + 2 * lq] = w[0];
+                out[2 + 2 * lq] = w[1];
             } else {
                 uint32_t w = 0;
                 if (!plain) {
@@ -244,11 +246,21 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restr
                     for (int i = 0; i < 8; ++i)
                         w |= (uint32_t)q4_code(__fadd_rn(__fmul_rn(x[u][i], id), 8.5f)) << (4 * i);
                 }
-                if (store) {
-                    reinterpret_cast<uint32_t *>(out + 4)[lq] = w;
-                    if (lq == 0) *reinterpret_cast<float *>(out) = d;
-                }
+                out[1 + lq] = w;
             }
+            if (lq == 0) out[0] = __float_as_uint(d);
+        }
+        // the run's bytes, contiguous, by whole lanes (this wave's own staging: LDS keeps a wave's
+        // accesses in order)
+        uint32_t *o = reinterpret_cast<uint32_t *>(dst + (size_t)r0 * BB);
+        if (wide && r0 + kRun <= nblocks) {
+#pragma unroll
+            for (int k = 0; k < (kWords / 4 + kWave - 1) / kWave; ++k)
+                if (k * kWave + lane < kWords / 4)
+                    reinterpret_cast<u32x4 *>(o)[k * kWave + lane] = reinterpret_cast<const u32x4 *>(mine)[k * kWave + lane];
+        } else {
+            const int words = (int)min((long)kRun, nblocks - r0) * (BB / 4);
+            for (int k = lane; k < words; k += kWave) o[k] = mine[k];
         }
     }
 }

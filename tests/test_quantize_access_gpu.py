@@ -11,15 +11,17 @@ pytestmark = pytest.mark.gpu
 
 
 def _run(dtype, src_dtype, src, lead):
-    """quantize with the source `lead` elements into its allocation."""
+    """quantize with the source `lead` elements into its allocation, and the blocks off 16 bytes."""
     from sapphire_amd.device import DeviceArray, check, lib
     m, k = src.shape
     flat = np.concatenate([np.zeros(lead, src.dtype), src.reshape(-1)])
     ds = DeviceArray.from_numpy(flat)
     nb = (k + 31) // 32
-    out = DeviceArray(m * nb * synth.BLOCK_BYTES[dtype])
-    check(lib().sapphire_quantize_dev(dtype, src_dtype, ds.ptr + lead * src.itemsize, m, k, out.ptr, None))
-    return np.frombuffer(out.numpy().tobytes(), synth.block_dtype(dtype)).reshape(m, nb)
+    at = 4 * (lead % 4)                                        # the blocks need 4-byte alignment only
+    out = DeviceArray(m * nb * synth.BLOCK_BYTES[dtype] + 16)
+    check(lib().sapphire_quantize_dev(dtype, src_dtype, ds.ptr + lead * src.itemsize, m, k, out.ptr + at, None))
+    raw = out.numpy().tobytes()[at:at + m * nb * synth.BLOCK_BYTES[dtype]]
+    return np.frombuffer(raw, synth.block_dtype(dtype)).reshape(m, nb)
 
 
 @pytest.mark.parametrize("dtype", [Q4, Q8], ids=["q4_0", "q8_0"])
