@@ -53,9 +53,13 @@ __global__ __launch_bounds__(kThreads) void prefill_qkv_kernel(PrefillAttn a, fl
 // their positions. The four waves take the piece's 16-position tiles in turn, each with a running
 // (max, sum, O) per row, merged at the end; the partial goes to a.part (O, unnormalised) and
 // a.ms (max in log2 units, sum). A piece without positions of its rows leaves (-inf, 0).
-// head_dim 256 keeps K, V and O of a tile in registers: one wave per SIMD, 512 of them.
+// Two register buffers of half a tile's K or V rows each are refilled as soon as they are used (K
+// low half, K high half, V of two positions per lane, V of the other two), so that with O a wave of
+// head_dim 256 stays under 256 registers and two waves share a SIMD. (Whole tiles of K and V took
+// 512, the moves between their two halves costing as much as the products: 48 us per layer of 1000
+// tokens, now 36.)
 template <int DPL, int G>
-__global__ __launch_bounds__(kThreads, DPL == 4 ? 1 : 2) void prefill_attn_kernel(PrefillAttn a, const float *__restrict__ q_rows) {
+__global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(PrefillAttn a, const float *__restrict__ q_rows) {
     constexpr int HD = kWave * DPL, NJ = HD / 16, TOK = kRows / G, LD = HD + 4;
     __shared__ __attribute__((aligned(16))) float buf[kWaves * kRows * LD];   // q, later the waves' O
     __shared__ float wm[kWaves][kRows], wsum[kWaves][kRows];
@@ -85,19 +89,23 @@ __global__ __launch_bounds__(kThreads, DPL == 4 ? 1 : 2) void prefill_attn_kerne
             q_rows + (size_t)min(t0 + r / G, tl) * nq + (hk * G + r % G) * HD + d);
     }
     const float *kc = a.kc + (size_t)hk * a.max_ctx * HD, *vc = a.vc + (size_t)hk * a.max_ctx * HD;
-    f4 kr[NJ], vr[4][DPL];
-    // rows past the piece repeat its last one (masked)
-    auto load_k = [&](int tb) {
-        const float *p = kc + (size_t)min(tb + c, hi - 1) * HD + 4 * m;
+    constexpr int HALF = NJ / 2;
+    static_assert(HALF == 2 * DPL, "half a tile's K rows and half its V rows are the same size");
+    f4 bufs[2][HALF];
+    // K of position tb + c, dims 16 j + 4 m .. + 3 for j in half h; positions past the piece repeat
+    // its last one (masked)
+    auto load_k = [&](int tb, int h) {
+        const float *p = kc + (size_t)min(tb + c, hi - 1) * HD + 4 * m + 16 * HALF * h;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) kr[j] = *reinterpret_cast<const f4 *>(p + 16 * j);
+        for (int j = 0; j < HALF; ++j) bufs[h][j] = *reinterpret_cast<const f4 *>(p + 16 * j);
     };
-    auto load_v = [&](int tb) {
+    // V of positions tb + 4 m + r, r = 2 h and 2 h + 1, dims 64 q + 4 c .. + 3
+    auto load_v = [&](int tb, int h) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float *p = vc + (size_t)min(tb + 4 * m + r, hi - 1) * HD + 4 * c;
+        for (int r = 0; r < 2; ++r) {
+            const float *p = vc + (size_t)min(tb + 4 * m + 2 * h + r, hi - 1) * HD + 4 * c;
 #pragma unroll
-            for (int q = 0; q < DPL; ++q) vr[r][q] = *reinterpret_cast<const f4 *>(p + 64 * q);
+            for (int q = 0; q < DPL; ++q) bufs[h][r * DPL + q] = *reinterpret_cast<const f4 *>(p + 64 * q);
         }
     };
     f4 o[DPL][4];                                      // o[q][e][r']: dim 64 q + 16 m + 4 r' + e of row c
@@ -108,18 +116,23 @@ __global__ __launch_bounds__(kThreads, DPL == 4 ? 1 : 2) void prefill_attn_kerne
     float mx = -INFINITY, sum = 0.f;                   // sum: this lane's positions only
     const float sl2 = __fmul_rn(a.scale, 1.44269504088896341f);
     int tb = lo + wid * kPos;
-    if (tb < hi) load_k(tb);
+    if (tb < hi) {
+        load_k(tb, 0);
+        load_k(tb, 1);
+    }
     __syncthreads();
     for (; tb < hi; tb += kWaves * kPos) {
-        load_v(tb);
         f4 s4[4] = {};
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const f4 qv = *reinterpret_cast<const f4 *>(buf + c * LD + 16 * j + 4 * m);
+        for (int h = 0; h < 2; ++h) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) s4[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[j][e], qv[e], s4[e], 0, 0, 0);
+            for (int j = 0; j < HALF; ++j) {
+                const f4 qv = *reinterpret_cast<const f4 *>(buf + c * LD + 16 * (HALF * h + j) + 4 * m);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s4[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(bufs[h][j][e], qv[e], s4[e], 0, 0, 0);
+            }
+            load_v(tb, h);
         }
-        if (tb + kWaves * kPos < hi) load_k(tb + kWaves * kPos);
         const f4 st = (s4[0] + s4[1]) + (s4[2] + s4[3]);
         float sc[4], mt = -INFINITY;
         bool on[4], edge = false;
@@ -154,37 +167,41 @@ __global__ __launch_bounds__(kThreads, DPL == 4 ? 1 : 2) void prefill_attn_kerne
         if (__any(edge)) {
             uint32_t ex = 0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int q = 0; q < DPL; ++q)
+                for (int j = 0; j < HALF; ++j)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) ex = max(ex, __float_as_uint(vr[r][q][e]) & 0x7f800000u);
+                    for (int e = 0; e < 4; ++e) ex = max(ex, __float_as_uint(bufs[h][j][e]) & 0x7f800000u);
             slow = __any(ex == 0x7f800000u) != 0;
         }
-        if (!slow) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
+        const int tn = tb + kWaves * kPos;
+        if (slow) {
+            for (int k = 0; k < kPos; ++k) {
+                const int t = tb + k;
+                const float pk = k & 2 ? (k & 1 ? p[3] : p[2]) : (k & 1 ? p[1] : p[0]);
+                const float w = __shfl(pk, (k >> 2) * 16 + c, kWave);
+                if (t < r_lo || t >= r_hi) continue;
+                const float *v = vc + (size_t)t * HD + 16 * m;
 #pragma unroll
                 for (int q = 0; q < DPL; ++q)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        o[q][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[r][q][e], p[r], o[q][e], 0, 0, 0);
-        } else {
+                    for (int r2 = 0; r2 < 4; ++r2)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                for (int mm = 0; mm < 4; ++mm) {
-                    const int t = tb + 4 * mm + r;
-                    const float w = __shfl(p[r], mm * 16 + c, kWave);
-                    if (t < r_lo || t >= r_hi) continue;
-                    const float *v = vc + (size_t)t * HD + 16 * m;
+                        for (int e = 0; e < 4; ++e)
+                            o[q][e][r2] = __builtin_fmaf(w, v[64 * q + 4 * r2 + e], o[q][e][r2]);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (!slow)
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
 #pragma unroll
                     for (int q = 0; q < DPL; ++q)
 #pragma unroll
-                        for (int r2 = 0; r2 < 4; ++r2)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                o[q][e][r2] = __builtin_fmaf(w, v[64 * q + 4 * r2 + e], o[q][e][r2]);
-                }
+                        for (int e = 0; e < 4; ++e)
+                            o[q][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(bufs[h][r * DPL + q][e], p[2 * h + r], o[q][e], 0, 0, 0);
+            load_k(tn, h);                             // past the end: the last row again
         }
     }
     sum += __shfl_xor(sum, 16, kWave);
