@@ -119,6 +119,11 @@ int run_staged(kernel_context_t *c, std::initializer_list<HostVec> ins, std::ini
     return 0;
 }
 
+// A GEMV result up to this long is stored straight into the pinned staging buffer by the kernel
+// (posted writes over the bus) instead of copied there by a second operation behind it: 2048 rows
+// 21.9 -> 20.6 us per call, 8192 32 -> 23, 16384 (64 KiB) 40 -> 31.
+constexpr size_t kDirectBytes = 64 << 10;
+
 // GEMV/GEMM core: Y[b*M + r] = A[r,:] . X[b*K ...] for b < batch.
 int gemv_exec(kernel_context_t *c, const tensor_t *A, const float *X, float *Y, int batch) {
     if (!c || !c->initialized) {
@@ -148,6 +153,8 @@ int gemv_exec(kernel_context_t *c, const tensor_t *A, const float *X, float *Y, 
     char *db = static_cast<char *>(c->d_stage);
     float *hx = reinterpret_cast<float *>(hb), *hy = reinterpret_cast<float *>(hb + align256(xb));
     float *dx = reinterpret_cast<float *>(db), *dy = reinterpret_cast<float *>(db + align256(xb));
+    const bool direct = batch == 1 && yb <= kDirectBytes;
+    if (direct) dy = hy;               // hipHostMalloc memory: the same address on the device
     for (int b = 0; b < batch; ++b) {
         memcpy(hx + (size_t)b * Kp, X + (size_t)b * K, sizeof(float) * (size_t)K);
         if (Kp > K) memset(hx + (size_t)b * Kp + K, 0, sizeof(float) * (size_t)(Kp - K));
@@ -168,7 +175,7 @@ int gemv_exec(kernel_context_t *c, const tensor_t *A, const float *X, float *Y, 
             rc = launch_gemv_f(dt, w, M, K, dx + (size_t)b * K, dy + (size_t)b * M, c->stream);
     }
     if (rc != 0) return -1;
-    if (!hip_ok(hipMemcpyAsync(hy, dy, yb, hipMemcpyDeviceToHost, c->stream), "D2H y")) return -1;
+    if (!direct && !hip_ok(hipMemcpyAsync(hy, dy, yb, hipMemcpyDeviceToHost, c->stream), "D2H y")) return -1;
     if (!hip_ok(hipStreamSynchronize(c->stream), "hipStreamSynchronize")) return -1;
     memcpy(Y, hy, yb);
     return 0;
