@@ -85,8 +85,8 @@ int sapphire_decoder_generate(sapphire_decoder_t *dec, int token, int pos, int s
  * decoder) run through every layer and leave their K/V rows in that sequence's cache, as
  * inference_forward_batch does for a prompt without logits (inference.c:236-244, 616-651:
  * every row of a chunk is written before its attention reads any, attention.c:292-309).
- * Chunks of up to 16 tokens run their projections as one matrix-core GEMM. No logits; the
- * next call is sapphire_decoder_generate with the prompt's last token at pos + n.
+ * Up to 16 tokens run as one chunk; longer prompts in passes of up to 1024 tokens, every
+ * weight read once per pass (matrix-core GEMMs, attention in fp32). No logits; the next call is sapphire_decoder_generate with the prompt's last token at pos + n.
  * Needs hidden, n_heads*head_dim and ffn multiples of 128 and hidden <= 1152 (-1
  * otherwise). elapsed_ms, if not NULL, receives the device time. 0 / -1. */
 int sapphire_decoder_prefill(sapphire_decoder_t *dec, int seq, const int *tokens, int n, int pos,

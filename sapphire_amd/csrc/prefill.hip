@@ -122,18 +122,24 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(PrefillAttn a
     }
     __syncthreads();
     for (; tb < hi; tb += kWaves * kPos) {
-        f4 s4[4] = {};
+        // a score is the sum of short chains (the weight's relative error is its absolute one)
+        constexpr int CH = HALF < 4 ? HALF : 4;
+        f4 st = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
 #pragma unroll
-            for (int j = 0; j < HALF; ++j) {
-                const f4 qv = *reinterpret_cast<const f4 *>(buf + c * LD + 16 * (HALF * h + j) + 4 * m);
+            for (int j0 = 0; j0 < HALF; j0 += CH) {
+                f4 s4[4] = {};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s4[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(bufs[h][j][e], qv[e], s4[e], 0, 0, 0);
+                for (int j = j0; j < j0 + CH; ++j) {
+                    const f4 qv = *reinterpret_cast<const f4 *>(buf + c * LD + 16 * (HALF * h + j) + 4 * m);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s4[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(bufs[h][j][e], qv[e], s4[e], 0, 0, 0);
+                }
+                st += (s4[0] + s4[1]) + (s4[2] + s4[3]);
             }
             load_v(tb, h);
         }
-        const f4 st = (s4[0] + s4[1]) + (s4[2] + s4[3]);
         float sc[4], mt = -INFINITY;
         bool on[4], edge = false;
 #pragma unroll
