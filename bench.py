@@ -138,7 +138,7 @@ def decode_leg(steps: int, cpu: bool, seed: int = 20260101, prefill: int = 1024)
     m = smodel.synthetic_model(smodel.GEMMA3_270M, seed)
     k, v = m.kv_prefill(prefill)
     out = bench_decode(steps, seed=seed, prefill=prefill, m=m, kv=(k, v))
-    # prefill of a 1024-token prompt into an empty cache (chunks of 16 through the batched GEMMs)
+    # prefill of a 1024-token prompt into an empty cache (one pass through the many-vector GEMMs)
     from sapphire_amd.engine import Decoder
     dec = Decoder(m)
     prompt = synth.rng(seed, 77).integers(0, m.cfg.vocab, prefill).astype(np.int32)
