@@ -145,6 +145,14 @@ __device__ __forceinline__ void shift_into_place(int e0, int K, float (&x)[8]) {
 // truncating rounds halves away from zero and everything else to the nearest.
 __device__ __forceinline__ int round_away(float v) { return (int)__fadd_rn(v, copysignf(0x1.fffffep-2f, v)); }
 
+// Between a wave's LDS stores and its other lanes' loads of them (and the next trip's stores): the
+// hardware keeps a wave's LDS accesses in order, the compiler reasons per lane and is told here.
+// No instruction of it is left in the kernel.
+__device__ __forceinline__ void wave_handover() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // DENSE: K % 32 == 0, so block b starts at element 32b. Otherwise row and block come from a
 // 32-bit division (the launcher keeps such matrices below 2^31 blocks).
 template <int DST, int SRC, int ACC, bool DENSE, int U>
@@ -250,8 +258,8 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restr
             }
             if (lq == 0) out[0] = __float_as_uint(d);
         }
-        // the run's bytes, contiguous, by whole lanes (this wave's own staging: LDS keeps a wave's
-        // accesses in order)
+        wave_handover();
+        // the run's bytes, contiguous, by whole lanes
         uint32_t *o = reinterpret_cast<uint32_t *>(dst + (size_t)r0 * BB);
         if (wide && r0 + kRun <= nblocks) {
 #pragma unroll
@@ -262,6 +270,7 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(const void *__restr
             const int words = (int)min((long)kRun, nblocks - r0) * (BB / 4);
             for (int k = lane; k < words; k += kWave) o[k] = mine[k];
         }
+        wave_handover();
     }
 }
 
