@@ -84,19 +84,19 @@ __device__ __forceinline__ float row16_scatter(const float (&a)[4], int n) {
 }
 
 // The MFMA B operand of this lane for group g (8 signed digits) and the factor
-// 2^(8d - sh) of its column. Lane l supplies column n = l % 16 (block j = n / 4 of the
+// 2^(8d - sh) of its column, from the lane's eight elements (lane_elems). Lane l supplies column n = l % 16 (block j = n / 4 of the
 // group, digit d = n % 4) for the k-slots of lane group m = l / 16: elements 8m..8m+7 of
 // block 4g + j, in the order the A operand holds them (natural for Q8_0; even then odd
 // elements for Q4_0, whose A bytes are the low nibbles, then the high nibbles).
 // NaN and infinite activations are zeroed here (nf is set): the row results get their fold
 // added when they are stored.
+__device__ __forceinline__ const float4 *lane_elems(const float *__restrict__ x, int g, int lane) {
+    return reinterpret_cast<const float4 *>(x + (4 * g + ((lane & 15) >> 2)) * 32 + 8 * (lane >> 4));
+}
 template <int DT>
-__device__ __forceinline__ void lane_digits(const float *__restrict__ x, int g, int lane, uint32_t &w0,
-                                            uint32_t &w1, float &p, bool &nf) {
-    const int n = lane & 15, m = lane >> 4;
-    const int j = n >> 2, d = n & 3;
-    const float4 *xp = reinterpret_cast<const float4 *>(x + (4 * g + j) * 32 + 8 * m);
-    const float4 va = xp[0], vb = xp[1];
+__device__ __forceinline__ void lane_digits(float4 va, float4 vb, int lane, uint32_t &w0, uint32_t &w1, float &p,
+                                            bool &nf) {
+    const int d = lane & 3;
     float v[8] = {va.x, va.y, va.z, va.w, vb.x, vb.y, vb.z, vb.w};
     int mexp = 0;
 #pragma unroll
@@ -297,7 +297,7 @@ __device__ __forceinline__ void tile_store(const float (&acc)[4], float *__restr
 // loads stays in flight in one tile of registers and two waves fit a SIMD. (Refilled a whole
 // tile at a time, or two tiles deep, those rows kept one wave per SIMD or waited for every tile.
 // 262144 rows with the softmax: Q4_0 K = 1152 48.8 -> 37.2 us, K = 1024 36.3 -> 33.7; Q8_0 61.1 ->
-// 56.2 and 56.1 -> 51.9. Three waves per SIMD instead of two spill and measured slower.) Each wave builds its B digits once. With kEpSoftmax every workgroup also leaves the softmax/argmax
+// 56.2 and 56.1 -> 51.9.) Each wave builds its B digits once. With kEpSoftmax every workgroup also leaves the softmax/argmax
 // partial of its rows in part[blockIdx.x] (folded by softmax_finish_parts). With
 // kEpGreedyStep every workgroup leaves the greedy key of its rows in its slot of gs.keys and
 // counts itself done; the last one takes the maximum key, decodes the token and advances the
@@ -330,10 +330,17 @@ __global__ __launch_bounds__(256, NG > 5 ? 2 : 1) void gemv_mfma(const uint8_t *
     float p[NG];
     long bop[NG];
     bool nfl = false;
+    float4 xv[NG][2];                                  // all in flight before the first is used: left
+                                                       // to the compiler, nine groups load in turn
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) xv[g][h] = lane_elems(x, g, lane)[h];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
         uint32_t w0, w1;
-        lane_digits<DT>(x, g, lane, w0, w1, p[g], nfl);
+        lane_digits<DT>(xv[g][0], xv[g][1], lane, w0, w1, p[g], nfl);
         bop[g] = (long)(((unsigned long)w1 << 32) | w0);
     }
     // the wave's lanes cover all of x
@@ -356,10 +363,10 @@ __global__ __launch_bounds__(256, NG > 5 ? 2 : 1) void gemv_mfma(const uint8_t *
             t += nwaves;
         }
     } else {
-        while (t < ntiles) {
-            // past the last tile the refills repeat it: the loads in flight, and so the waits,
-            // are the same in every trip
-            const int tn = min(t + nwaves, ntiles - 1);
+        // The last tile is multiplied apart, with nothing to refill: most waves have one to three
+        // tiles below 131072 rows, and a refill past the last one costs as much as another tile
+        // (Q8_0 32768 x 1152 11.6 us with it, 9.9 without; Q4_0 16384 x 1152 6.3 and 6.2).
+        auto multiply = [&](auto refill) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[r] = 0.f;
 #pragma unroll
@@ -368,12 +375,16 @@ __global__ __launch_bounds__(256, NG > 5 ? 2 : 1) void gemv_mfma(const uint8_t *
                 asm volatile("" : "+v"(bop[g]));
                 group_mfma<DT, NG>(RA, bop[g], p[g], g, lane, acc);
                 asm volatile("" ::: "memory");
-                group_issue<DT, NG>(RA, rq, rs, tn, g, lane);
-                asm volatile("" ::: "memory");
+                refill(g);
             }
             tile_store<DT, EP>(acc, y, M, t, lane, sp, key, nc);
-            t += nwaves;
-        }
+        };
+        for (; t + nwaves < ntiles; t += nwaves)
+            multiply([&](int g) {
+                group_issue<DT, NG>(RA, rq, rs, t + nwaves, g, lane);
+                asm volatile("" ::: "memory");
+            });
+        if (t < ntiles) multiply([](int) {});
     }
     if constexpr (EP == kEpGreedyStep) {
         key = lanes::u64_wave_max(key);
@@ -603,7 +614,10 @@ int cus_of_current_device() {
 // Waves per CU of the TILED GEMV. Measured on the 262144 x 640 LM head with cold weights:
 // Q8_0 (11.5 KiB per tile) is fastest at 8 (two per SIMD, its register limit for the double
 // buffer anyway), Q4_0 (6.4 KiB per tile, half the bytes per wave) at 12 (3 %).
-// Rows of more than five groups are bound to two waves per SIMD by their registers.
+// Longer Q8_0 rows are bound to two waves per SIMD by their registers (193-213). Longer Q4_0 rows
+// would fit three (141-159): 12 waves per CU take 262144 rows of K = 1152 in 29.5 us against 31.0
+// (K = 1024 27.0 and 28.1), but 65536 rows, whose tiles then no longer come out even, in 12.6
+// against 11.2 (11.3 and 10.2), so they keep 8 too.
 constexpr int kWavesPerCu = 8, kWavesPerCuShortQ4 = 12;
 
 unsigned tiled_blocks(int dt, int M, int K) {
