@@ -40,6 +40,7 @@ constexpr int kGroups = kSub / kGroup;          // groups per sub-chunk: one per
 static_assert(kGroup == 16 * kPer && kGroups == 16, "a group is a row of 16 lanes of the grid kernels");
 constexpr int kMaxSubs = 2048;                  // n <= 2^21 keeps the error bound below 1/4
 constexpr int kSlots = 12;                      // sub-chunks a walk fetches ahead
+constexpr int kShortSubs = 4;                   // rows up to this long take the walk with little LDS
 constexpr int kCap = 1 << 28;                   // saturation of map increments
 constexpr int kZero = -1000, kSub_ = -127;      // binade ids of 0 and of the subnormals
 
@@ -406,16 +407,21 @@ __global__ __launch_bounds__(kThreads) void smp_maps(const float *__restrict__ w
 // group where the same happens, and its elements are added one by one; the scan resumes after it.
 // The sub-chunks expected to hold a change (cross) are brought into LDS by four waves before the
 // walk, in one memory round trip instead of one each (37 -> 31 us per walk of 262144 weights).
+// SUBS, SLOTS: the sub-chunks of the longest row and those fetched ahead. The maps and elements of
+// kMaxSubs and kSlots fill most of a CU's LDS, so that 256 rows walk at a time; short rows come in
+// larger batches and take a form of which seven share a CU (draws from 300 rows of 64: 38 us, 71 with
+// the long form; 300 rows of 4096 77 and 115).
+template <int SUBS, int SLOTS>
 __global__ __launch_bounds__(kThreads) void smp_walk(const float *__restrict__ w, int n, size_t ldw, int chain,
                                                      int nsub, const SubMaps *__restrict__ maps,
                                                      const SubMaps *__restrict__ gmaps, const int *__restrict__ cross,
                                                      RowInfo *__restrict__ rows, const float *__restrict__ draws,
                                                      const int *__restrict__ d_step, int batch,
                                                      int *__restrict__ tokens) {
-    __shared__ SubMaps cm[kMaxSubs];
-    __shared__ float xs[kSlots + 1][kSub];             // the last slot: sub-chunks not fetched ahead
-    __shared__ SubMaps gs[kSlots + 1][kGroups];
-    __shared__ int slot_q[kSlots], nslots;
+    __shared__ SubMaps cm[SUBS];
+    __shared__ float xs[SLOTS + 1][kSub];              // the last slot: sub-chunks not fetched ahead
+    __shared__ SubMaps gs[SLOTS + 1][kGroups];
+    __shared__ int slot_q[SLOTS], nslots;
     const int b = blockIdx.x, lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     const RowInfo ri = rows[b];
     if (ri.bad) {
@@ -430,10 +436,10 @@ __global__ __launch_bounds__(kThreads) void smp_walk(const float *__restrict__ w
             const bool c = k + lane < nsub && cross[(size_t)b * nsub + k + lane] != 0;
             const unsigned long long bal = __ballot(c);
             const int at = have + __popcll(bal & ((1ull << lane) - 1));
-            if (c && at < kSlots) slot_q[at] = k + lane;
+            if (c && at < SLOTS) slot_q[at] = k + lane;
             have += __popcll(bal);
         }
-        if (lane == 0) nslots = min(have, kSlots);
+        if (lane == 0) nslots = min(have, SLOTS);
     } else {
         for (int k = threadIdx.x - kWave; k < nsub; k += kThreads - kWave) cm[k] = maps[(size_t)b * nsub + k];
     }
@@ -477,8 +483,8 @@ __global__ __launch_bounds__(kThreads) void smp_walk(const float *__restrict__ w
         // sub-chunk q: lane g < 16 holds group g's maps
         const int base = q * kSub;
         const unsigned long long hit = __ballot(my_q == q);
-        const int slot = hit ? first_lane(hit) : kSlots;
-        if (!hit) fetch(kSlots, q);
+        const int slot = hit ? first_lane(hit) : SLOTS;
+        if (!hit) fetch(SLOTS, q);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // one wave: its LDS accesses are in order
         const SubMaps gm = gs[slot][lane & (kGroups - 1)];
         int from = 0;                                  // the first group not yet added
@@ -594,16 +600,15 @@ int launch_sample(const float *logits, int n, int batch, size_t ld, float temper
     hipLaunchKernelGGL(smp_weights, grid, dim3(kThreads), 0, s, logits, n, ld, inv_t, scale, temperature, w, ldw,
                        stats, rows);
     if (!hip_ok(hipGetLastError(), "sample weights launch")) return -1;
-    hipLaunchKernelGGL(smp_maps, grid, dim3(kThreads), 0, s, w, n, ldw, 0, stats, rows, maps, gmaps, cross);
-    if (!hip_ok(hipGetLastError(), "sample maps launch")) return -1;
-    hipLaunchKernelGGL(smp_walk, dim3(batch), dim3(kThreads), 0, s, w, n, ldw, 0, nsub, maps, gmaps, cross, rows, draws, d_step,
-                       batch, tokens);
-    if (!hip_ok(hipGetLastError(), "sample sum walk launch")) return -1;
-    hipLaunchKernelGGL(smp_maps, grid, dim3(kThreads), 0, s, w, n, ldw, 1, stats, rows, maps, gmaps, cross);
-    if (!hip_ok(hipGetLastError(), "sample maps launch")) return -1;
-    hipLaunchKernelGGL(smp_walk, dim3(batch), dim3(kThreads), 0, s, w, n, ldw, 1, nsub, maps, gmaps, cross, rows, draws, d_step,
-                       batch, tokens);
-    return hip_ok(hipGetLastError(), "sample draw walk launch") ? 0 : -1;
+    auto walk = nsub <= kShortSubs ? smp_walk<kShortSubs, kShortSubs> : smp_walk<kMaxSubs, kSlots>;
+    for (int chain = 0; chain < 2; ++chain) {
+        hipLaunchKernelGGL(smp_maps, grid, dim3(kThreads), 0, s, w, n, ldw, chain, stats, rows, maps, gmaps, cross);
+        if (!hip_ok(hipGetLastError(), "sample maps launch")) return -1;
+        hipLaunchKernelGGL(walk, dim3(batch), dim3(kThreads), 0, s, w, n, ldw, chain, nsub, maps, gmaps, cross, rows, draws,
+                           d_step, batch, tokens);
+        if (!hip_ok(hipGetLastError(), "sample walk launch")) return -1;
+    }
+    return 0;
 }
 
 }  // namespace sapphire

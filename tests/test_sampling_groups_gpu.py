@@ -24,3 +24,18 @@ def test_draws_at_group_edges(L, oracle, n, shape):
     for j, r in enumerate(draws):
         hit = np.flatnonzero(cum >= r)
         assert toks[j] == (int(hit[0]) if hit.size else n - 1), (j, float(r))
+
+
+@pytest.mark.parametrize("n", [4096, 4097])
+def test_many_rows_of_each_walk(L, oracle, n):
+    """The longest row of the walk that shares a CU and the shortest of the other, in more rows than
+    there are CUs: every row its own draw."""
+    g = np.random.default_rng(n)
+    row = (g.standard_normal(n) * 3).astype(np.float32)
+    _, w = oracle.sample(row, 1.0, 0.5)
+    s = np.add.accumulate(w, dtype=np.float32)[-1]
+    cum = np.add.accumulate(w / s, dtype=np.float32)
+    draws = np.concatenate([g.random(298, np.float32), cum[[1023, 4095]]]).astype(np.float32)
+    toks, _ = _gpu_sample(L, np.tile(np.concatenate([row, np.zeros(PAD, np.float32)]), (draws.size, 1)), n, 1.0, draws)
+    want = [int(np.argmax(cum >= r)) if (cum >= r).any() else n - 1 for r in draws]
+    assert toks.tolist() == want
