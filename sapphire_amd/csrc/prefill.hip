@@ -158,7 +158,8 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(PrefillAttn a
         sum = __fmul_rn(sum, f);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            p[r] = on[r] ? __builtin_amdgcn_exp2f(sc[r] - mn) : 0.f;
+            // masked, or a score of -inf (also where every score so far is, mn included)
+            p[r] = sc[r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sc[r] - mn);
             sum = __fadd_rn(sum, p[r]);
         }
         mx = mn;
@@ -220,7 +221,8 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_attn_kernel(PrefillAttn a
     float top = wm[0][c];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) top = fmaxf(top, wm[w][c]);
-    // a wave without positions of the row has sum 0 and O 0; its factor must not be NaN
+    // a wave without positions of the row, or with scores of -inf only, has sum 0 and O 0; its
+    // factor must not be NaN
     const float fw = sum == 0.f ? 0.f : __builtin_amdgcn_exp2f(mx - top);
     float *mine = buf + (size_t)(wid * kRows + c) * LD + 16 * m;
 #pragma unroll

@@ -78,3 +78,41 @@ def test_long_prompt_non_finite_token(oracle, bad):
         assert fin[:, :, :at].all() and not fin[:, :, at].all()
         assert np.array_equal(np.isfinite(got), fin), f"{what}: non-finite rows differ"
         assert np.abs(got[fin] - ref[fin]).max() <= 2e-3 * np.abs(ref[fin]).max()
+
+
+def test_long_prompt_cached_keys_without_weight(oracle):
+    """Cached keys whose scores are -inf (a run of them that fills a tile of 16 positions) have
+    weight 0 and spoil nothing. One dim of the keys is infinite, with the sign against the two
+    query heads': a dim that hardly turns with the position, found by trying them on the oracle."""
+    from sapphire_amd.engine import Decoder
+    cfg = _cfg(n_layers=2, n_heads=4, n_kv_heads=2, head_dim=64, sliding_window=1000, global_layers=(0, 1))
+    kv0, n = 64, 20
+    m = smodel.synthetic_model(cfg, 63)
+    k0, v0 = m.kv_prefill(kv0)
+    prompt = np.full(n, 7, np.int32)              # one token: its queries differ by their position only
+    rows = slice(kv0, kv0 + n)
+
+    def with_inf(signs):
+        k = k0.copy()
+        for h, (d, s) in enumerate(signs):
+            if d is not None:
+                k[0, h, 16:32, d] = s * np.inf
+        return k
+
+    def reference(signs):
+        rk, rv = with_inf(signs), v0.copy()
+        oracle_prefill(oracle, m, rk, rv, prompt, kv0, nthreads=4)
+        return rk, rv, np.isfinite(rk[1, :, rows]).all() and np.isfinite(rv[1, :, rows]).all()
+
+    tries = [(d, s) for d in range(63, 47, -1) for s in (1, -1)]
+    none = (None, 0)
+    signs = [next(t for t in tries if reference([t, none])[2]), next(t for t in tries if reference([none, t])[2])]
+    rk, rv, finite = reference(signs)
+    assert finite
+    dec = Decoder(m)
+    dec.set_kv(with_inf(signs), v0)
+    dec.prefill(prompt, kv0)
+    gk, gv = dec.get_kv()
+    dec.close()
+    _kv_close(gk, rk, rows, "K")
+    _kv_close(gv, rv, rows, "V")
