@@ -62,7 +62,12 @@ typedef struct {
 
 typedef struct sapphire_decoder sapphire_decoder_t;
 
-/* Uploads the weights to the current device (NULL on error; sapphire_last_error()). */
+/* Uploads the weights to the current device (NULL on error; sapphire_last_error()). Besides the
+ * weights, the cache and the step's buffers a decoder whose shapes sapphire_decoder_prefill takes
+ * holds buffers for passes of up to 1024 prompt tokens (75 MB for the Gemma-3-270M shape, 122 MB for
+ * the 1B shape), and a one-sequence decoder the prefill's copy of the projections (62 MB for the
+ * 270M shape in Q4_0). Where the prompt buffers find no room, creation succeeds and prompts run in
+ * chunks of 16 tokens. */
 sapphire_decoder_t *sapphire_decoder_create(const sapphire_decoder_config_t *cfg,
                                             const sapphire_decoder_weights_t *w);
 void sapphire_decoder_destroy(sapphire_decoder_t *dec);
@@ -86,7 +91,10 @@ int sapphire_decoder_generate(sapphire_decoder_t *dec, int token, int pos, int s
  * inference_forward_batch does for a prompt without logits (inference.c:236-244, 616-651:
  * every row of a chunk is written before its attention reads any, attention.c:292-309).
  * Up to 16 tokens run as one chunk; longer prompts in passes of up to 1024 tokens, every
- * weight read once per pass (matrix-core GEMMs, attention in fp32). No logits; the next call is sapphire_decoder_generate with the prompt's last token at pos + n.
+ * weight read once per pass (matrix-core GEMMs, attention in fp32). The two forms add in different
+ * orders: a token's K/V rows agree to fp32 rounding, not bit for bit, between a call of up to 16
+ * tokens and a longer one. No logits; the next call is sapphire_decoder_generate with the prompt's
+ * last token at pos + n.
  * Needs hidden, n_heads*head_dim and ffn multiples of 128 and hidden <= 1152 (-1
  * otherwise). elapsed_ms, if not NULL, receives the device time. 0 / -1. */
 int sapphire_decoder_prefill(sapphire_decoder_t *dec, int seq, const int *tokens, int n, int pos,

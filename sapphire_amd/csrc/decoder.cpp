@@ -120,7 +120,8 @@ struct sapphire_decoder {
     float *pf_dparts = nullptr, *pf_dout = nullptr, *pf_part = nullptr;
     int *pf_tok = nullptr;       // [kPrefillChunk] tokens, then [kPrefillChunk] positions
     // longer prompts: passes of up to wp_tokens tokens through the many-vector GEMMs (gemm_wide.h)
-    // and the prompt attention (prefill.h); 0 when the shapes do not fit them
+    // and the prompt attention (prefill.h); 0 when the shapes do not fit them or the buffers found
+    // no room
     int wp_tokens = 0;
     float *wp_resid[2] = {nullptr, nullptr};
     float *wp_qkv = nullptr, *wp_q = nullptr, *wp_part = nullptr, *wp_o = nullptr, *wp_g = nullptr, *wp_down = nullptr;
@@ -873,6 +874,42 @@ bool valid_batch_config(const sapphire_decoder_config_t &c, int batch) {
 
 bool setup_persistent(sapphire_decoder *d);
 
+// The buffers of long prompts (75 MB for the Gemma-3-270M shape, 122 MB for the 1B shape, at 1024
+// tokens a pass). Made with the decoder, so that no prompt waits for them; a decoder that finds no
+// room for them still runs every prompt, in chunks of 16.
+void alloc_prompt_buffers(sapphire_decoder *d) {
+    const auto &c = d->cfg;
+    const int H = c.hidden, hd = c.head_dim, nq = c.n_heads * hd, nk = c.n_kv_heads * hd;
+    if (!d->pf_ok || !prefill_attn_supported(c.n_heads, c.n_kv_heads, hd) || !gemm_wide_supported(H) ||
+        !gemm_wide_supported(nq) || !gemm_wide_supported(c.ffn) || c.max_ctx < kWideMinTokens)
+        return;
+    const int T = std::min(kWideTokens, c.max_ctx);
+    const size_t t = (size_t)T, rows = t * c.n_heads * kPrefillPieces;
+    // a product's result, or the partial sums of its K splits
+    const size_t hp = std::max(t * H, gemm_wide_parts_bytes(H, T) / sizeof(float));
+    const size_t ob = std::max({gemm_wide_operand_bytes(T, H), gemm_wide_operand_bytes(T, nq),
+                                gemm_wide_operand_bytes(T, c.ffn)});
+    char *const cur = d->arena_cur;
+    const size_t left = d->arena_left, chunks = d->allocs.size();
+    if (dev_alloc_t(d, &d->wp_resid[0], t * H, "prompt resid") &&
+        dev_alloc_t(d, &d->wp_resid[1], t * H, "prompt resid") &&
+        dev_alloc_t(d, &d->wp_qkv, t * (nq + 2 * nk), "prompt qkv") && dev_alloc_t(d, &d->wp_q, t * nq, "prompt q") &&
+        dev_alloc_t(d, &d->wp_part, rows * hd, "prompt attention partials") &&
+        dev_alloc_t(d, &d->wp_ms, rows, "prompt attention maxima") && dev_alloc_t(d, &d->wp_o, hp, "prompt o") &&
+        dev_alloc_t(d, &d->wp_g, t * c.ffn, "prompt g") && dev_alloc_t(d, &d->wp_down, hp, "prompt down") &&
+        dev_alloc(d, &d->wp_op, ob, "prompt operands") && dev_alloc_t(d, &d->wp_tok, c.max_ctx, "prompt tokens")) {
+        d->wp_tokens = T;
+        return;
+    }
+    (void)hipGetLastError();                           // handled here: not the next launch's error
+    while (d->allocs.size() > chunks) {
+        (void)hipFree(d->allocs.back());
+        d->allocs.pop_back();
+    }
+    d->arena_cur = cur;
+    d->arena_left = left;
+}
+
 sapphire_decoder_t *create_decoder(const sapphire_decoder_config_t *cfg, const sapphire_decoder_weights_t *w,
                                    int batch) {
     if (!cfg || !w) {
@@ -1101,24 +1138,7 @@ sapphire_decoder_t *create_decoder(const sapphire_decoder_config_t *cfg, const s
             !dev_alloc_t(d, &d->pf_tok, 2 * p, "prefill tokens"))
             return fail();
     }
-    if (d->pf_ok && prefill_attn_supported(c.n_heads, c.n_kv_heads, hd) && gemm_wide_supported(H) &&
-        gemm_wide_supported(nq) && gemm_wide_supported(c.ffn) && c.max_ctx >= kWideMinTokens) {
-        const int T = std::min(kWideTokens, c.max_ctx);
-        const size_t t = (size_t)T, rows = t * c.n_heads * kPrefillPieces;
-        // a product's result, or the partial sums of its K splits
-        const size_t hp = std::max(t * H, gemm_wide_parts_bytes(H, T) / sizeof(float));
-        const size_t ob = std::max({gemm_wide_operand_bytes(T, H), gemm_wide_operand_bytes(T, nq),
-                                    gemm_wide_operand_bytes(T, c.ffn)});
-        if (!dev_alloc_t(d, &d->wp_resid[0], t * H, "prompt resid") ||
-            !dev_alloc_t(d, &d->wp_resid[1], t * H, "prompt resid") ||
-            !dev_alloc_t(d, &d->wp_qkv, t * (nq + 2 * nk), "prompt qkv") || !dev_alloc_t(d, &d->wp_q, t * nq, "prompt q") ||
-            !dev_alloc_t(d, &d->wp_part, rows * hd, "prompt attention partials") ||
-            !dev_alloc_t(d, &d->wp_ms, rows, "prompt attention maxima") || !dev_alloc_t(d, &d->wp_o, hp, "prompt o") ||
-            !dev_alloc_t(d, &d->wp_g, t * c.ffn, "prompt g") || !dev_alloc_t(d, &d->wp_down, hp, "prompt down") ||
-            !dev_alloc(d, &d->wp_op, ob, "prompt operands") || !dev_alloc_t(d, &d->wp_tok, c.max_ctx, "prompt tokens"))
-            return fail();
-        d->wp_tokens = T;
-    }
+    alloc_prompt_buffers(d);
     if (B == 1 && !setup_persistent(d)) return fail();
     // the zero fills above run on the null stream; the decoder's stream does not wait for it
     if (!hip_ok(hipDeviceSynchronize(), "hipDeviceSynchronize")) return fail();
