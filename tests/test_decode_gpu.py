@@ -436,8 +436,8 @@ def _kv_close(got, ref, sl, what):
 
 
 @pytest.mark.parametrize("cfg,seed,kv0,n,steps", [
-    (smodel.TINY, 41, 0, 40, 8),       # chunks 16 + 16 + 8, local layers slide while prefilling
-    (MID, 42, 20, 37, 10),             # on top of 20 cached positions; chunks 16 + 16 + 5
+    (smodel.TINY, 41, 0, 40, 8),       # local layers slide while prefilling
+    (MID, 42, 20, 37, 10),             # on top of 20 cached positions
     (smodel.GEMMA3_270M, 43, 0, 100, 16),
 ], ids=["tiny", "mid_on_cache", "gemma3_270m"])
 def test_prefill_matches_oracle(oracle, cfg, seed, kv0, n, steps):
