@@ -14,7 +14,9 @@ bool gemm_wide_supported(int K);
 size_t gemm_wide_operand_bytes(int T, int K);
 // K splits a launch with out.parts takes: parts holds splits * T * M floats.
 int gemm_wide_splits(int dt, int M, int K, int T);
-// Bytes of those at most.
+// Weight rows of its workgroups' tile.
+int gemm_wide_tile_rows(int dt, int M, int K, int T);
+// Bytes of the partial sums at most.
 size_t gemm_wide_parts_bytes(int M, int T);
 // The operands of T tokens from `in` (GemmIn's transform, sums of squares as trees).
 int launch_gemm_wide_prep(int dt, const GemmIn &in, int K, int T, void *operand, hipStream_t s);

@@ -509,6 +509,12 @@ int gemm_wide_splits(int dt, int M, int K, int T) {
     return k;
 }
 
+int gemm_wide_tile_rows(int dt, int M, int K, int T) {
+    int s, k;
+    plan(dt, M, K, T, true, &s, &k);
+    return kShapes[s].bn;
+}
+
 int launch_gemm_wide_prep(int dt, const GemmIn &in, int K, int T, void *operand, hipStream_t st) {
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
     if (!gemm_wide_supported(K) || T <= 0 || !operand || in.x_blocked || (!in.x && !in.parts) ||

@@ -6,9 +6,12 @@ Tolerance: an output is a float32 sum of K products in chunks, each product with
 of at most 2^-21 (two fp16 terms), so |error| <= (2^-21 + 2 sqrt(K) 2^-24) sum |w x| with room for
 the order of the sums; a wrong or missing product is of the order of sum |w x| / K.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
+import sapphire_amd
 from sapphire_amd import synth
 from tests.test_gemm_gpu import TILED, _gemm, _ref
 from tests.test_nonfinite_gpu import _matrix, _patterns, _same_special
@@ -23,7 +26,7 @@ CASES = [                 # m, k, batch
     (1152, 6912, 100),    # K split, chunks cut by the split
     (129, 8192, 31),      # the longest K
     (130, 8320, 20),      # past it: passes of 16
-    (4111, 640, 512),     # the 128- and 256-row tiles, one full pass
+    (4111, 640, 512),     # the 256-row tile (Q8_0: 128), one full pass
     (8192, 256, 300),
     (384, 384, 513),      # two passes, the second of one token
 ]
@@ -44,6 +47,60 @@ def test_gemm_wide(hip, dtype, m, k, batch):
     ref, mag = X.astype(np.float64) @ w.T, np.abs(X.astype(np.float64)) @ np.abs(w).T
     bound = (2.0 ** -21 + 2.0 * np.sqrt(k) * 2.0 ** -24) * mag
     assert np.all(np.abs(got - ref) <= bound), f"worst {np.max(np.abs(got - ref) / np.maximum(bound, 1e-300)):.2f} of the bound"
+
+
+def _plan(dtype, m, k, tokens):
+    """(rows of the workgroup tile, K splits) that the library chooses on this device."""
+    lib = ctypes.CDLL(sapphire_amd.LIB_PATH)         # C++ functions of the library, not of its API
+    return tuple(getattr(lib, f"_ZN8sapphire{len(n)}{n}Eiiii")(dtype, m, k, tokens)
+                 for n in ("gemm_wide_tile_rows", "gemm_wide_splits"))
+
+
+def test_cases_reach_every_tile(hip):
+    """The shapes above and below, on 256 CUs: each (dtype, tile) instance, its K splits, and beside
+    the 64-row tile also K past the two-level sums' (2304)."""
+    want = {
+        (640, 2048, 64): [(64, True), (64, True)],
+        (4111, 640, 512): [(256, False), (128, False)],
+        (8192, 256, 300): [(256, False), (128, False)],
+        (2305, 1152, 500): [(128, False), (128, False)],
+        (4111, 2560, 300): [(128, False), (128, False)],
+        (1152, 6912, 100): [(64, True), (64, True)],
+    }
+    for (m, k, t), tiles in want.items():
+        for dtype, (rows, split) in zip((synth.Q4_0, synth.Q8_0), tiles):
+            got = _plan(dtype, m, k, t)
+            assert (got[0], got[1] > 1) == (rows, split), f"{m}x{k} {t} tokens dtype {dtype}: {got}"
+    assert set(want) <= set(CASES) | set(TILE_CASES)
+
+
+TILE_CASES = [            # the 128-row tile of both dtypes, ragged in rows and tokens
+    (2305, 1152, 500),
+    (4111, 2560, 300),    # K past the two-level sums of the 256-row tile
+]
+
+
+@pytest.mark.parametrize("dtype", [synth.Q4_0, synth.Q8_0], ids=["q4_0", "q8_0"])
+@pytest.mark.parametrize("m,k,batch", TILE_CASES, ids=lambda v: str(v))
+def test_gemm_wide_128_row_tile(hip, dtype, m, k, batch):
+    test_gemm_wide(hip, dtype, m, k, batch)
+
+
+@pytest.mark.parametrize("dtype", [synth.Q4_0, synth.Q8_0], ids=["q4_0", "q8_0"])
+@pytest.mark.parametrize("m,k,batch", [(2305, 1152, 500), (4111, 640, 512)], ids=lambda v: str(v))
+def test_gemm_wide_non_finite_in_larger_tiles(hip, oracle, dtype, m, k, batch):
+    """Special values in the 128- and 256-row tiles: in their own vectors' rows, and nowhere else."""
+    from sapphire_amd.device import QMatrix
+    W = _matrix(dtype, m, k, 55)
+    X = synth.normal_f32((batch, k), 55, 5)
+    at = (0, 33, 64, batch - 1)
+    for b, x in zip(at, _patterns(k, 56).values()):
+        X[b] = x
+    got = _gemm(hip, QMatrix(dtype, W, layout=TILED), X)
+    ref = _ref(oracle, dtype, W, X[list(at)])
+    for i, b in enumerate(at):
+        _same_special(got[b], ref[i])
+    assert np.isfinite(np.delete(got, at, axis=0)).all()
 
 
 @pytest.mark.parametrize("dtype", [synth.Q4_0, synth.Q8_0], ids=["q4_0", "q8_0"])
