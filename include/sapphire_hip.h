@@ -99,7 +99,10 @@ int sapphire_gemm_bf16_dev(const void *w, int M, int K, const float *x, int ldx,
  * fp16 matrix cores, up to 16 sequences in one pass and longer batches in passes of 512, with
  * `ws` holding sapphire_gemm_workspace_bytes(dtype, M, K) bytes of device memory (K-split
  * partial sums, prepared activations); calls that share a workspace must be ordered on one stream. On AOS/PACKED it is
- * the vector kernel and ws may be NULL. */
+ * the vector kernel and ws may be NULL. A vector's result does not depend on the others; on
+ * the TILED layout its bits do not depend on `batch` up to 16 either, while above it the tile and
+ * K split, and with them the order of the fp32 sums, follow M, K and batch, so that the result
+ * agrees with that of another batch to fp32 rounding. */
 size_t sapphire_gemm_workspace_bytes(int dtype, int M, int K);
 int sapphire_gemm_q_dev(int dtype, int layout, const void *w, int M, int K, const float *X, int batch,
                         float *Y, void *ws, void *stream);

@@ -104,17 +104,17 @@ struct Unit {
 
 // Loads of unit (tile, group) gb: the lane's 16 (or 2 x 16) quant bytes and row n's four
 // block scales. The unit offset is wave-uniform (scalar offset), the lane part constant.
-template <int DT, int AUX = kNT>
+template <int DT>
 __device__ __forceinline__ void unit_issue(Unit &u, __amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rs,
                                            uint32_t gb, int lane, int n) {
     constexpr int NQ = DT == DT_Q8_0 ? 2 : 1;
 #pragma unroll
     for (int h = 0; h < NQ; ++h)
-        u.a[h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, lane * 16u + h * 1024u, gb * (NQ * 1024u), AUX));
+        u.a[h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, lane * 16u + h * 1024u, gb * (NQ * 1024u), kNT));
     if constexpr (NQ == 1) u.a[1] = u.a[0];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-        u.s[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, n * 4u + j * 64u, gb * 256u, AUX));
+        u.s[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, n * 4u + j * 64u, gb * 256u, kNT));
 }
 
 struct BConst {

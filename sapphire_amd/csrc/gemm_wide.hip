@@ -6,12 +6,14 @@
 //
 // Two launches: gemm_wide_prep_kernel forms the A operands of every token once, in the order
 // in which the matrix cores read them (2 KiB per 16 tokens and block: hi, lo); gemm_wide_kernel
-// brings them into LDS by DMA (no registers, two stages of four blocks) and every workgroup
+// brings them into LDS by DMA (no registers; three stages of four blocks, two for the larger stages
+// of Q4_0's 256-row and Q8_0's 128-row tile) and every workgroup
 // multiplies BM tokens by BN weight rows, so that a weight is read and expanded once per BM
 // tokens instead of once per 16. Q4_0 6912 x 1152 x 300: 166 us in passes of 16 (19 of them,
 // each reading all the weights and bound by its staging and latency) -> 29 us.
 #include "gemm_body.h"
 #include "gemm_wide.h"
+#include "prefill.h"
 
 namespace sapphire {
 
@@ -47,7 +49,6 @@ Operand operand_at(void *buf, int T, int K) {
     return o;
 }
 
-constexpr int kAttnPieces = 8;
 struct AttnParts {
     const float *part;             // [pieces][T][nh][hd], unnormalised
     const float2 *ms;              // [pieces][T][nh]: maximum (log2 units), sum
@@ -127,10 +128,10 @@ __global__ __launch_bounds__(kThreads) void gemm_wide_prep_kernel(GemmIn in, int
             const int nh = K / at.hd, h = p * 8 / at.hd, d = p * 8 - h * at.hd;
             const size_t row = (size_t)t * nh + h, rows = (size_t)gridDim.x * nh;
             // every piece's loads first; a piece without positions (-inf, 0) has no O
-            float2 ms[kAttnPieces];
-            float ov[kAttnPieces][8];
+            float2 ms[kPrefillPieces];
+            float ov[kPrefillPieces][8];
 #pragma unroll
-            for (int c = 0; c < kAttnPieces; ++c) {
+            for (int c = 0; c < kPrefillPieces; ++c) {
                 ms[c] = make_float2(-INFINITY, 0.f);
                 if (c < at.pieces) {
                     ms[c] = at.ms[c * rows + row];
@@ -139,10 +140,10 @@ __global__ __launch_bounds__(kThreads) void gemm_wide_prep_kernel(GemmIn in, int
             }
             float top = -INFINITY, sum = 0.f;
 #pragma unroll
-            for (int c = 0; c < kAttnPieces; ++c)
+            for (int c = 0; c < kPrefillPieces; ++c)
                 if (ms[c].y != 0.f) top = fmaxf(top, ms[c].x);
 #pragma unroll
-            for (int c = 0; c < kAttnPieces; ++c)
+            for (int c = 0; c < kPrefillPieces; ++c)
                 if (ms[c].y != 0.f) {
                     const float f = __builtin_amdgcn_exp2f(ms[c].x - top);
                     sum = __fadd_rn(sum, __fmul_rn(ms[c].y, f));
@@ -251,7 +252,6 @@ __device__ float token_fold(const Operand &op, int flags, const uint8_t *__restr
 struct WideArgs {
     const uint8_t *wq;
     const uint8_t *wsc;
-    uint32_t q_bytes, s_bytes;
     Operand op;
     int M, K, T;
     int nt, nm, ks;                // workgroup tiles over the tokens / the rows, K splits
@@ -263,24 +263,24 @@ struct WideArgs {
 
 static_assert(kChunk == 8 * kGroupBlocks, "a chunk's range scale covers 8 groups");
 
-// One workgroup of NWN x NWT waves: wave (wn, wt) multiplies WT tiles of 16 tokens by WN tiles
-// of 16 weight rows. A stage is one TILED group (four blocks) of the workgroup's operands,
+// One workgroup of NW waves: each multiplies the workgroup's WT tiles of 16 tokens by WN tiles of 16
+// weight rows of its own. A stage is one TILED group (four blocks) of the workgroup's operands,
 // weights and scales, brought into LDS by DMA (no registers in flight) D - 1 groups ahead. One
 // barrier per group: a stage is refilled after the barrier that ends its reads.
 // The sums run in three levels (a group, a chunk, the row) so that no fp32 chain is longer than
 // the K chunks and wave shares of the 16-vector GEMM make it there; four row tiles per wave
 // leave registers for two (two groups, the row), enough up to kMaxTwoLevelK.
-template <int DT, int WN, int WT, int NWN, int NWT, int D>
-__global__ __launch_bounds__(NWN *NWT *kWave, 2) void gemm_wide_kernel(WideArgs p) {
-    constexpr int NW = NWN * NWT, NQ = DT == DT_Q8_0 ? 2 : 1;
-    constexpr int BT = WT * NWT, BN = WN * NWN;        // tiles of 16 tokens / rows
-    constexpr int kA = BT * 8 * 1024, kQ = BN * NQ * 1024, kS = BN * 256, kStage = kA + kQ + kS;
-    constexpr int kDma = BT * 8 / NW + BN * (NQ + 1) / NW;   // DMA instructions of a wave per stage
-    static_assert(BT * 8 % NW == 0 && BN % NW == 0, "every wave issues the same number");
+template <int DT, int WN, int WT, int NW, int D>
+__global__ __launch_bounds__(NW *kWave, 2) void gemm_wide_kernel(WideArgs p) {
+    constexpr int NQ = DT == DT_Q8_0 ? 2 : 1;
+    constexpr int BN = WN * NW;                        // tiles of 16 rows
+    constexpr int kA = WT * 8 * 1024, kQ = BN * NQ * 1024, kS = BN * 256, kStage = kA + kQ + kS;
+    constexpr int kDma = WT * 8 / NW + BN * (NQ + 1) / NW;   // DMA instructions of a wave per stage
+    static_assert(WT * 8 % NW == 0 && BN % NW == 0, "every wave issues the same number");
     __shared__ __attribute__((aligned(16))) char lds[D][kStage];
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wid = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int wn = wid % NWN, wt = wid / NWN, n = lane & 15, m = lane >> 4;
+    const int n = lane & 15, m = lane >> 4;
     // Workgroups go to the XCDs round robin: each XCD takes a contiguous range of the tiles, so
     // that its L2 holds one side's share once instead of both sides whole.
     const int total = gridDim.x, per = total / kXcds, rem = total % kXcds, xcd = blockIdx.x % kXcds;
@@ -301,9 +301,9 @@ __global__ __launch_bounds__(NWN *NWT *kWave, 2) void gemm_wide_kernel(WideArgs 
     auto issue = [&](int slot, int g) {
         char *st = lds[slot];
 #pragma unroll
-        for (int i = 0; i < BT * 8 / NW; ++i) {        // a tile of 16 tokens: 8 KiB in one piece
+        for (int i = 0; i < WT * 8 / NW; ++i) {        // a tile of 16 tokens: 8 KiB in one piece
             const int c = i * NW + wid;
-            dma16(p.op.a + ((size_t)(bt * BT + (c >> 3)) * nb + g * kGroupBlocks) * 2 * kWave + (c & 7) * kWave + lane,
+            dma16(p.op.a + ((size_t)(bt * WT + (c >> 3)) * nb + g * kGroupBlocks) * 2 * kWave + (c & 7) * kWave + lane,
                   st + c * 1024);
         }
 #pragma unroll
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(NWN *NWT *kWave, 2) void gemm_wide_kernel(WideArgs 
         Unit u[WN];
 #pragma unroll
         for (int i = 0; i < WN; ++i) {
-            const int c = wn * WN + i;
+            const int c = wid * WN + i;
 #pragma unroll
             for (int h = 0; h < NQ; ++h) u[i].a[h] = *reinterpret_cast<const u32x4 *>(st + kA + (c * NQ + h) * 1024 + lane * 16);
 #pragma unroll
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(NWN *NWT *kWave, 2) void gemm_wide_kernel(WideArgs 
             for (int j = 0; j < JB; ++j)
 #pragma unroll
                 for (int q = 0; q < WT; ++q) {
-                    const h8 *a = x + ((wt * WT + q) * kGroupBlocks + j0 + j) * 2 * kWave + lane;
+                    const h8 *a = x + (q * kGroupBlocks + j0 + j) * 2 * kWave + lane;
                     hi[j][q] = a[0];
                     lo[j][q] = a[kWave];
                 }
@@ -389,7 +389,7 @@ __global__ __launch_bounds__(NWN *NWT *kWave, 2) void gemm_wide_kernel(WideArgs 
         if (g == g0 || (g & 7) == 0)
 #pragma unroll
             for (int j = 0; j < WT; ++j)
-                sc[j] = *reinterpret_cast<const f4 *>(p.op.xsc + (size_t)(g >> 3) * p.op.tokens + ((bt * NWT + wt) * WT + j) * 16 + 4 * m);
+                sc[j] = *reinterpret_cast<const f4 *>(p.op.xsc + (size_t)(g >> 3) * p.op.tokens + (bt * WT + j) * 16 + 4 * m);
         asm volatile("" ::: "memory");
         issue(slot == 0 ? D - 1 : slot - 1, min(g + D - 1, g1 - 1));
         multiply(lds[slot]);
@@ -425,14 +425,14 @@ __global__ __launch_bounds__(NWN *NWT *kWave, 2) void gemm_wide_kernel(WideArgs 
     int4 flags[WT];                                    // padded tokens': read, not used
 #pragma unroll
     for (int q = 0; q < WT; ++q)
-        flags[q] = *reinterpret_cast<const int4 *>(p.op.flag + ((bt * NWT + wt) * WT + q) * 16 + 4 * m);
+        flags[q] = *reinterpret_cast<const int4 *>(p.op.flag + (bt * WT + q) * 16 + 4 * m);
     float *dst = p.y + (p.ks > 1 ? (size_t)kz * p.T * p.M : 0);
 #pragma unroll
     for (int q = 0; q < WT; ++q) {
-        const int t0 = (bt * BT + wt * WT + q) * 16 + 4 * m;
+        const int t0 = (bt * WT + q) * 16 + 4 * m;
 #pragma unroll
         for (int i = 0; i < WN; ++i) {
-            const int ti = bm * BN + wn * WN + i, row = ti * kTileRows + n;
+            const int ti = bm * BN + wid * WN + i, row = ti * kTileRows + n;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 float val = tot[i][q][r];
@@ -469,14 +469,17 @@ constexpr int kNumShapes = 3, kSmallest = kNumShapes - 1;
 constexpr int kMaxTwoLevelK = 2304;
 constexpr int kSplitPerCu = 2;     // workgroups per CU up to which K is split
 
-// The workgroup tile and K split of a GEMM. An A operand read from LDS feeds the MFMAs of the
-// rows of one wave, and those reads are what bounds the kernel, so the widest tile that still
-// gives every CU a workgroup is the fastest (Q4_0 16384 x 6912 x 512: 278 us at 256 rows, 309 at
-// 128, 385 at 64; 640 x 1024 x 512, where only the last one covers the CUs: 20, 15 and 12 us;
-// Q8_0's 256-row stage leaves one workgroup per CU and loses). Where the smallest tile leaves
-// CUs idle, K is split until two workgroups per CU: 1152 x 6912 x 300 takes 37 us in two parts
-// against 48 (three per CU: 640 x 2048 x 500 23 us against 20, the partial sums' traffic), but 640 x 1024 x 300 12.7 against 12.0, the partial sums costing more than the
-// shorter chains save, so not below 12 groups.
+// The workgroup tile and K split of a GEMM. An A operand read from LDS feeds the MFMAs of the rows of
+// one wave, so a wider tile has fewer LDS reads and waits per product, and the widest one that still
+// gives every CU a workgroup is the fastest (Q4_0 16384 x 6912 x 512: 278 us at 256 rows, 309 at 128,
+// 385 at 64; 640 x 1024 x 512, where only the last one covers the CUs: 20, 15 and 12 us; Q8_0's
+// 256-row stage leaves one workgroup per CU and loses). The last round of workgroups is not looked
+// at: just past the CUs (Q4_0 6912 x 1152: 288 tokens, 243 workgroups, 21.7 us; 300 tokens, 270 of
+// them, 30.7) every tile takes the same (30.8, 30.0 and 30.0 us). Where the smallest tile leaves CUs
+// idle, K is split until two workgroups per CU: 1152 x 6912 x 300 takes 37 us in two parts against 48
+// (three per CU: 640 x 2048 x 500 23 us against 20, the partial sums' traffic), but 640 x 1024 x 300
+// 12.7 against 12.0, the partial sums costing more than the shorter chains save, so not below 12
+// groups.
 void plan(int dt, int M, int K, int T, bool may_split, int *shape, int *ks) {
     const int cus = cu_count(), G = K / (kGroupBlocks * kBlock);
     auto grid = [&](int i) { return ((T + kShapes[i].bm - 1) / kShapes[i].bm) * ((M + kShapes[i].bn - 1) / kShapes[i].bn); };
@@ -536,7 +539,7 @@ int launch_gemm_wide_prep(int dt, const GemmIn &in, int K, int T, void *operand,
 int launch_gemm_wide_prep_attn(int dt, const float *part, const void *ms, int pieces, int nh, int hd, int T,
                                void *operand, hipStream_t st) {
     const int K = nh * hd;
-    if (!gemm_wide_supported(K) || K > 8 * kThreads || T <= 0 || pieces < 1 || pieces > kAttnPieces || hd % 8 != 0) {
+    if (!gemm_wide_supported(K) || K > 8 * kThreads || T <= 0 || pieces < 1 || pieces > kPrefillPieces || hd % 8 != 0) {
         set_error("wide GEMM attention input: unsupported arguments (T=%d, %d heads of %d, %d pieces)", T, nh, hd, pieces);
         return -1;
     }
@@ -559,8 +562,6 @@ int launch_gemm_wide(int dt, const void *w, int M, int K, int T, const void *ope
     WideArgs a;
     a.wq = static_cast<const uint8_t *>(w);
     a.wsc = a.wq + so;
-    a.q_bytes = (uint32_t)so;
-    a.s_bytes = (uint32_t)(q_tiled_bytes(dt, M, K) - so);
     a.op = operand_at(const_cast<void *>(operand), T, K);
     a.M = M;
     a.K = K;
@@ -575,11 +576,11 @@ int launch_gemm_wide(int dt, const void *w, int M, int K, int T, const void *ope
     a.geglu = out.geglu;
     const dim3 grid((unsigned)(a.nt * a.nm * ks));
     // stages: as many as leave two workgroups per CU
-    if (dt == DT_Q4_0 && s == 0) hipLaunchKernelGGL((gemm_wide_kernel<DT_Q4_0, 4, 2, 4, 1, 2>), grid, dim3(256), 0, st, a);
-    else if (dt == DT_Q4_0 && s == 1) hipLaunchKernelGGL((gemm_wide_kernel<DT_Q4_0, 2, 2, 4, 1, 3>), grid, dim3(256), 0, st, a);
-    else if (dt == DT_Q4_0) hipLaunchKernelGGL((gemm_wide_kernel<DT_Q4_0, 1, 2, 4, 1, 3>), grid, dim3(256), 0, st, a);
-    else if (s == 1) hipLaunchKernelGGL((gemm_wide_kernel<DT_Q8_0, 2, 2, 4, 1, 2>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((gemm_wide_kernel<DT_Q8_0, 1, 2, 4, 1, 3>), grid, dim3(256), 0, st, a);
+    if (dt == DT_Q4_0 && s == 0) hipLaunchKernelGGL((gemm_wide_kernel<DT_Q4_0, 4, 2, 4, 2>), grid, dim3(256), 0, st, a);
+    else if (dt == DT_Q4_0 && s == 1) hipLaunchKernelGGL((gemm_wide_kernel<DT_Q4_0, 2, 2, 4, 3>), grid, dim3(256), 0, st, a);
+    else if (dt == DT_Q4_0) hipLaunchKernelGGL((gemm_wide_kernel<DT_Q4_0, 1, 2, 4, 3>), grid, dim3(256), 0, st, a);
+    else if (s == 1) hipLaunchKernelGGL((gemm_wide_kernel<DT_Q8_0, 2, 2, 4, 2>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((gemm_wide_kernel<DT_Q8_0, 1, 2, 4, 3>), grid, dim3(256), 0, st, a);
     return hip_ok(hipGetLastError(), "gemm_wide launch") ? 0 : -1;
 }
 
