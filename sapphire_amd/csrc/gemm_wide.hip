@@ -474,8 +474,9 @@ constexpr int kSplitPerCu = 2;     // workgroups per CU up to which K is split
 // gives every CU a workgroup is the fastest (Q4_0 16384 x 6912 x 512: 278 us at 256 rows, 309 at 128,
 // 385 at 64; 640 x 1024 x 512, where only the last one covers the CUs: 20, 15 and 12 us; Q8_0's
 // 256-row stage leaves one workgroup per CU and loses). The last round of workgroups is not looked
-// at: just past the CUs (Q4_0 6912 x 1152: 288 tokens, 243 workgroups, 21.7 us; 300 tokens, 270 of
-// them, 30.7) every tile takes the same (30.8, 30.0 and 30.0 us). Where the smallest tile leaves CUs
+// at: just past the CUs every tile takes the same (Q4_0 6912 x 1152 x 300, 270 workgroups of 256
+// rows: 30.8 us, 128 rows 30.0, 64 rows 30.0; 288 tokens, where 243 would not cover the CUs: 23.8,
+// 21.9 and 25.2). Where the smallest tile leaves CUs
 // idle, K is split until two workgroups per CU: 1152 x 6912 x 300 takes 37 us in two parts against 48
 // (three per CU: 640 x 2048 x 500 23 us against 20, the partial sums' traffic), but 640 x 1024 x 300
 // 12.7 against 12.0, the partial sums costing more than the shorter chains save, so not below 12
